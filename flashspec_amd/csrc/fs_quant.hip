@@ -6,6 +6,8 @@
 // Contraction is disabled so `x / scale + zero` keeps its two roundings; division is the
 // correctly rounded HIP default.  One wavefront quantizes one [rows, head_dim] group.
 
+#include <type_traits>
+
 #include "fs_common.h"
 
 #pragma clang fp contract(off)
@@ -111,10 +113,12 @@ __device__ __forceinline__ void quantize_any_group(const Get& get, int rows, int
 }
 
 // ---- vectorized group quantizer --------------------------------------------------------------
-// Same arithmetic as quantize_group, for a group of `rows` contiguous source rows of D values
-// with rows*D = CH*512 and D % 8 == 0: lane l holds values [c*512 + 8l, c*512 + 8l + 8) of
-// every chunk c in registers, read once from HBM with 16-byte loads (non-temporal: the source
-// is read exactly once) and written back as 8-byte packed int8 stores.
+// Same arithmetic as quantize_group, for a group of `rows` contiguous source rows of D values with
+// D % 8 == 0 and n = rows*D <= CH*512: lane l holds values [c*512 + 8l, c*512 + 8l + 8) of every
+// chunk c in registers, read once from HBM with 16-byte loads (non-temporal: the source is read
+// exactly once) and written back as 8-byte packed stores.  Lanes past the group's n values (head
+// dims such as 80, whose groups are no multiple of 512) hold its first eight again, which leaves
+// the extremes as they are, and store nothing.
 
 typedef uint32_t q_u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -153,7 +157,7 @@ __device__ __forceinline__ void load8(const __hip_bfloat16* p, float* f) {
 // Quantize CH chunks of 8 values held by this lane and store them as packed bytes.
 template <int CH, bool RCP>
 __device__ __forceinline__ void store_chunks(const float (&x)[CH][8], float scale, float rcp, float zero,
-                                             int8_t* dst, int lane) {
+                                             int8_t* dst, int n, int lane) {
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     uint32_t w[2] = {0u, 0u};
@@ -165,25 +169,28 @@ __device__ __forceinline__ void store_chunks(const float (&x)[CH][8], float scal
       w[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(qv, i % 4, w[i / 4]);
     }
     // stored as q - 128: flip the top bit of every byte
-    *(uint2*)(dst + c * 512 + lane * 8) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+    const int e = c * 512 + lane * 8;
+    if (e < n) *(uint2*)(dst + e) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
   }
 }
 
 // One lane's share of a vectorized group as loaded: CH chunks of 8 source values (16 bytes each
-// for 16-bit types, 32 for fp32); chunks past the group's valid rows are zero.
+// for 16-bit types, 32 for fp32); values past the group's valid ones are zero.
 template <int CH, typename XT>
 struct RawGroup {
   static constexpr int kWords = sizeof(XT) == 4 ? 2 * CH : CH;
   q_u32x4_t w[kWords];
 };
 
+// `valid`: the group's values that exist in the source, `n` its values with the zero rows.
 template <int CH, typename XT>
-__device__ __forceinline__ void load_raw(RawGroup<CH, XT>& r, const XT* src, int valid_rows, int D, int lane) {
+__device__ __forceinline__ void load_raw(RawGroup<CH, XT>& r, const XT* src, int valid, int n, int lane) {
   constexpr int per = RawGroup<CH, XT>::kWords / CH;  // 16-byte words per chunk
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = c * 512 + lane * 8;
-    const bool ok = e / D < valid_rows;
+    const int at = c * 512 + lane * 8;
+    const int e = at < n ? at : 0;
+    const bool ok = e < valid;
 #pragma unroll
     for (int i = 0; i < per; ++i)
       r.w[c * per + i] = ok ? nt_load16((const char*)(src + e) + 16 * i) : q_u32x4_t{0u, 0u, 0u, 0u};
@@ -217,7 +224,7 @@ __device__ __forceinline__ void unpack8(const q_u32x4_t* w, const __hip_bfloat16
 // Quantizes a group held in registers (quantize_group's float32 op sequence).
 template <int CH>
 __device__ __forceinline__ void quantize_regs(const float (&x)[CH][8], int8_t* dst, float* scale_out,
-                                              int16_t* zero_out, int lane) {
+                                              int16_t* zero_out, int n, int lane) {
   float mn = __builtin_huge_valf(), mx = -__builtin_huge_valf();
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
@@ -236,9 +243,9 @@ __device__ __forceinline__ void quantize_regs(const float (&x)[CH][8], int8_t* d
   // |x| <= max(|mn|, |mx|) for every value of the group, and rounding is monotonic: if the
   // largest product is finite, all are (wave-uniform test)
   if (__builtin_isfinite(fmaxf(fabsf(mn), fabsf(mx)) * rcp))
-    store_chunks<CH, true>(x, scale, rcp, zero, dst, lane);
+    store_chunks<CH, true>(x, scale, rcp, zero, dst, n, lane);
   else
-    store_chunks<CH, false>(x, scale, rcp, zero, dst, lane);
+    store_chunks<CH, false>(x, scale, rcp, zero, dst, n, lane);
   if (lane == 0) {
     *scale_out = scale;
     *zero_out = (int16_t)zero;
@@ -250,16 +257,6 @@ __device__ __forceinline__ void unpack_group(const RawGroup<CH, XT>& r, float (&
   constexpr int per = RawGroup<CH, XT>::kWords / CH;
 #pragma unroll
   for (int c = 0; c < CH; ++c) unpack8(&r.w[c * per], (const XT*)nullptr, x[c]);
-}
-
-template <int CH, typename XT>
-__device__ __forceinline__ void quantize_group_vec(const XT* src, int valid_rows, int D, int8_t* dst,
-                                                   float* scale_out, int16_t* zero_out, int lane) {
-  RawGroup<CH, XT> r;
-  load_raw(r, src, valid_rows, D, lane);
-  float x[CH][8];
-  unpack_group(r, x);
-  quantize_regs<CH>(x, dst, scale_out, zero_out, lane);
 }
 
 // Where group `grp` of a vectorized quantize pass reads and writes.
@@ -275,25 +272,26 @@ struct GroupRef {
 // Waves loop over groups grp = wave, wave + waves, ...: the next group's loads are issued before
 // the current group is quantized, so every wave keeps a group's bytes in flight while it computes.
 template <int CH, typename XT, typename Map>
-__device__ __forceinline__ void quantize_groups_pipelined(const Map& map, int64_t ngroups, int D) {
+__device__ __forceinline__ void quantize_groups_pipelined(const Map& map, int64_t ngroups, int rows, int D) {
   const int lane = threadIdx.x & (kWave - 1);
+  const int n = rows * D;
   const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
   int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   if (grp >= ngroups) return;
   GroupRef<XT> cur = map(grp);
   RawGroup<CH, XT> raw;
-  load_raw(raw, cur.src, cur.valid_rows, D, lane);
+  load_raw(raw, cur.src, cur.valid_rows * D, n, lane);
   for (;;) {
     const int64_t nxt = grp + waves;
     GroupRef<XT> ref_next{};
     RawGroup<CH, XT> raw_next;
     if (nxt < ngroups) {
       ref_next = map(nxt);
-      load_raw(raw_next, ref_next.src, ref_next.valid_rows, D, lane);
+      load_raw(raw_next, ref_next.src, ref_next.valid_rows * D, n, lane);
     }
     float x[CH][8];
     unpack_group(raw, x);
-    quantize_regs<CH>(x, cur.dst, cur.scale, cur.zero, lane);
+    quantize_regs<CH>(x, cur.dst, cur.scale, cur.zero, n, lane);
     if (nxt >= ngroups) break;
     grp = nxt;
     cur = ref_next;
@@ -301,7 +299,15 @@ __device__ __forceinline__ void quantize_groups_pipelined(const Map& map, int64_
   }
 }
 
-// Chunks of 512 values per group when the vectorized quantizer applies, else 0.
+// 512-value chunks of a group of `rows` rows when the vectorized quantizers apply (rounded up to an
+// instantiated count), else 0.
+static int group_chunks(int64_t rows, int D) {
+  if (D % 8 != 0 || rows * D > 8 * 512) return 0;
+  const int ch = (int)((rows * D + 511) / 512);
+  return ch == 5 ? 6 : (ch == 7 ? 8 : ch);
+}
+
+// Chunks of 512 values per group when the vectorized append applies, else 0.
 __host__ __device__ constexpr int vec_chunks(int rows, int D) {
   return (D % 8 == 0 && (rows * D) % 512 == 0 && rows * D / 512 <= 8) ? rows * D / 512 : 0;
 }
@@ -314,10 +320,10 @@ quantize_blocks_vec_kernel(const XT* x, int64_t outer, int S, int D, int bs, int
   auto map = [=](int64_t grp) {
     const int64_t o = grp / nb;
     const int blk = (int)(grp - o * nb);
-    return GroupRef<XT>{x + ((size_t)o * S + (size_t)blk * bs) * D, S - blk * bs, values + (size_t)grp * bs * D,
+    return GroupRef<XT>{x + ((size_t)o * S + (size_t)blk * bs) * D, min(S - blk * bs, bs), values + (size_t)grp * bs * D,
                         scale + grp, zero + grp};
   };
-  quantize_groups_pipelined<CH, XT>(map, outer * nb, D);
+  quantize_groups_pipelined<CH, XT>(map, outer * nb, bs, D);
 }
 
 // dense [B, H, S, D] -> page store [P, H, page, D], vectorized and pipelined (see
@@ -334,10 +340,10 @@ quantize_pages_vec_kernel(const XT* x, int H, int S, int D, int page, int nbps, 
     const unsigned o = page_src ? (unsigned)page_src[j] : j;
     const unsigned b = o / (unsigned)nbps;
     const int lb = (int)(o - b * (unsigned)nbps);
-    return GroupRef<XT>{x + (((size_t)(b * H + h) * S) + (size_t)lb * page) * D, S - lb * page,
+    return GroupRef<XT>{x + (((size_t)(b * H + h) * S) + (size_t)lb * page) * D, min(S - lb * page, page),
                         values + (size_t)grp * page * D, scale + grp, zero + grp};
   };
-  quantize_groups_pipelined<CH, XT>(map, P * H, D);
+  quantize_groups_pipelined<CH, XT>(map, P * H, page, D);
 }
 
 // x [outer, S, D] -> values [outer, nb, bs, D]; group = (o, block); rows past S read as 0.
@@ -421,6 +427,63 @@ struct PageStore {
   float* scale;
   int16_t* zero;
 };
+
+// Prompt admission (see fs_write_prompt_i8): one request's K and V rows [H, src_tokens, D] into the
+// pages of a store, group = (K or V, logical page, head).  The page ids travel in the launch's
+// arguments, so admitting a prompt needs no device copy of its page list: the reference-shaped path
+// (fs_update_pages_i8, one launch per tensor) uploaded a page list, a row map and a flag per page
+// for each tensor, six blocking copies of ~3.6 us, and read every source value twice.  Bound by HBM
+// (read 2 B, write 1 B per value).  Measured on MI355X, 3001 tokens, H32 D128 fp16, 49 MB read and
+// 25 MB written: the whole add_request 298 us -> 17.1 us (two element-wise kernels of 56 us before).
+constexpr int kPromptPages = 896;  // page ids per launch: 3.5 KiB of the 4 KiB argument limit
+struct PromptPages {
+  int32_t id[kPromptPages];
+};
+
+template <typename XT>
+struct PromptSource {
+  const XT* k;
+  const XT* v;
+  PageStore ks, vs;
+  int H, src_tokens, length, D, page;
+  int first, n;  // logical pages [first, first + n)
+};
+
+// Group grp of a prompt's pages: K groups first, then V groups, heads innermost (a page's heads are
+// consecutive in the store).
+template <typename XT>
+__device__ __forceinline__ GroupRef<XT> prompt_group(const PromptSource<XT>& s, const PromptPages& pages,
+                                                     int64_t grp) {
+  const unsigned per = (unsigned)s.n * (unsigned)s.H;
+  unsigned g = __builtin_amdgcn_readfirstlane((unsigned)grp);  // one group per wave
+  const bool second = g >= per;
+  if (second) g -= per;
+  const unsigned i = g / (unsigned)s.H;
+  const unsigned h = g - i * (unsigned)s.H;
+  const int row0 = (s.first + (int)i) * s.page;
+  const PageStore st = second ? s.vs : s.ks;
+  const size_t og = (size_t)pages.id[i] * s.H + h;
+  return GroupRef<XT>{(second ? s.v : s.k) + ((size_t)h * s.src_tokens + row0) * s.D,
+                      min(s.length - row0, s.page), st.values + og * s.page * s.D, st.scale + og, st.zero + og};
+}
+
+template <int CH, typename XT>
+__global__ void __launch_bounds__(256)
+prompt_pages_vec_kernel(const PromptSource<XT> s, int64_t groups, const PromptPages pages) {
+  auto map = [&](int64_t grp) { return prompt_group(s, pages, grp); };
+  quantize_groups_pipelined<CH, XT>(map, groups, s.page, s.D);
+}
+
+template <typename XT>
+__global__ void __launch_bounds__(256)
+prompt_pages_kernel(const PromptSource<XT> s, int64_t groups, const PromptPages pages) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  if (grp >= groups) return;
+  const GroupRef<XT> ref = prompt_group(s, pages, grp);
+  auto get = [&](int r, int d) -> float { return r < ref.valid_rows ? to_f32(ref.src[(size_t)r * s.D + d]) : 0.0f; };
+  quantize_group(get, s.page, s.D, ref.dst, ref.scale, ref.zero, lane);
+}
 
 // The advanced length of request b after its token at `pos` was stored (ok) or dropped; a dropped
 // token also counts into *dropped when the caller gave a counter.
@@ -526,9 +589,9 @@ append_tokens_vec_kernel(const XT* k_new, const XT* v_new, PageStore ks, PageSto
   const float zero = fminf(fmaxf(__builtin_rintf(-mn / scale), 0.0f), 255.0f);
   const float rcp = 1.0f / scale;
   if (__builtin_isfinite(fmaxf(fabsf(mn), fabsf(mx)) * rcp))
-    store_chunks<CH, true>(x, scale, rcp, zero, vals, lane);
+    store_chunks<CH, true>(x, scale, rcp, zero, vals, CH * 512, lane);
   else
-    store_chunks<CH, false>(x, scale, rcp, zero, vals, lane);
+    store_chunks<CH, false>(x, scale, rcp, zero, vals, CH * 512, lane);
   if (lane == 0) {
     st.scale[sidx] = scale;
     st.zero[sidx] = (int16_t)zero;
@@ -644,18 +707,31 @@ static dim3 vec_grid(int64_t groups) {
 
 static bool is_pow2_chunks(int ch) { return ch == 1 || ch == 2 || ch == 4 || ch == 8; }
 
-template <typename XT>
-static int launch_vec_blocks(int ch, dim3 grid, hipStream_t st, const XT* x, int64_t outer, int S, int D, int bs,
-                             int nb, int8_t* values, float* scale, int16_t* zero) {
-  const dim3 block(256);
+// f(integral_constant<CH>) for the instantiated chunk counts of group_chunks.
+template <typename F>
+static void by_chunks(int ch, F&& f) {
   switch (ch) {
-    case 1: hipLaunchKernelGGL((quantize_blocks_vec_kernel<1, XT>), grid, block, 0, st, x, outer, S, D, bs, nb, values, scale, zero); break;
-    case 2: hipLaunchKernelGGL((quantize_blocks_vec_kernel<2, XT>), grid, block, 0, st, x, outer, S, D, bs, nb, values, scale, zero); break;
-    case 4: hipLaunchKernelGGL((quantize_blocks_vec_kernel<4, XT>), grid, block, 0, st, x, outer, S, D, bs, nb, values, scale, zero); break;
-    default: hipLaunchKernelGGL((quantize_blocks_vec_kernel<8, XT>), grid, block, 0, st, x, outer, S, D, bs, nb, values, scale, zero); break;
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    default: f(std::integral_constant<int, 8>{}); break;
   }
-  return check_launch("quantize_int8_per_block");
 }
+
+// f(typed null pointer) for a source dtype code; false for an unknown code.
+template <typename F>
+static bool by_dtype(int dtype, F&& f) {
+  switch (dtype) {
+    case FS_F32: f((const float*)nullptr); return true;
+    case FS_F16: f((const __half*)nullptr); return true;
+    case FS_BF16: f((const __hip_bfloat16*)nullptr); return true;
+    default: return false;
+  }
+}
+template <typename T>
+using value_of = std::remove_cv_t<std::remove_pointer_t<T>>;
 
 template <typename XT>
 static int launch_vec_append(int ch, dim3 grid, hipStream_t st, const XT* k_new, const XT* v_new, PageStore ks,
@@ -672,19 +748,6 @@ static int launch_vec_append(int ch, dim3 grid, hipStream_t st, const XT* k_new,
   return check_launch("append_tokens");
 }
 
-template <typename XT>
-static int launch_vec_pages(int ch, dim3 grid, hipStream_t st, const XT* x, int H, int S, int D, int page, int nbps,
-                            const int64_t* page_src, int64_t P, int8_t* values, float* scale, int16_t* zero) {
-  const dim3 block(256);
-  switch (ch) {
-    case 1: hipLaunchKernelGGL((quantize_pages_vec_kernel<1, XT>), grid, block, 0, st, x, H, S, D, page, nbps, page_src, P, values, scale, zero); break;
-    case 2: hipLaunchKernelGGL((quantize_pages_vec_kernel<2, XT>), grid, block, 0, st, x, H, S, D, page, nbps, page_src, P, values, scale, zero); break;
-    case 4: hipLaunchKernelGGL((quantize_pages_vec_kernel<4, XT>), grid, block, 0, st, x, H, S, D, page, nbps, page_src, P, values, scale, zero); break;
-    default: hipLaunchKernelGGL((quantize_pages_vec_kernel<8, XT>), grid, block, 0, st, x, H, S, D, page, nbps, page_src, P, values, scale, zero); break;
-  }
-  return check_launch("quantize_pages");
-}
-
 }  // namespace fs
 
 using namespace fs;
@@ -698,23 +761,19 @@ extern "C" int fs_quantize_i8(const void* x, int x_dtype, int64_t outer, int seq
   const int64_t groups = outer * nb;
   if ((groups + 3) / 4 > 0x7fffffffLL) return set_error(FS_ERR_INVALID, "quantize: too many groups");
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  const int ch = vec_chunks(block_size, head_dim);
-  if (is_pow2_chunks(ch) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0) {
-    switch (x_dtype) {
-      case FS_F32: return launch_vec_blocks<float>(ch, vec_grid(groups), st, (const float*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
-      case FS_F16: return launch_vec_blocks<__half>(ch, vec_grid(groups), st, (const __half*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
-      case FS_BF16: return launch_vec_blocks<__hip_bfloat16>(ch, vec_grid(groups), st, (const __hip_bfloat16*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
-      default: return set_error(FS_ERR_INVALID, "quantize: dtype code must be 0, 1 or 2");
-    }
-  }
-  switch (x_dtype) {
-    case FS_F32: hipLaunchKernelGGL(quantize_blocks_kernel<float>, grid, block, 0, st, (const float*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero); break;
-    case FS_F16: hipLaunchKernelGGL(quantize_blocks_kernel<__half>, grid, block, 0, st, (const __half*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero); break;
-    case FS_BF16: hipLaunchKernelGGL(quantize_blocks_kernel<__hip_bfloat16>, grid, block, 0, st, (const __hip_bfloat16*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero); break;
-    default: return set_error(FS_ERR_INVALID, "quantize: dtype code must be 0, 1 or 2");
-  }
-  return check_launch("quantize_int8_per_block");
+  const int ch = ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 ? group_chunks(block_size, head_dim) : 0;
+  const bool known = by_dtype(x_dtype, [&](auto tag) {
+    using XT = value_of<decltype(tag)>;
+    const XT* src = (const XT*)x;
+    if (ch == 0)
+      hipLaunchKernelGGL(quantize_blocks_kernel<XT>, wave_grid(groups), dim3(256), 0, st, src, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
+    else
+      by_chunks(ch, [&](auto c) {
+        hipLaunchKernelGGL((quantize_blocks_vec_kernel<decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
+      });
+  });
+  return known ? check_launch("quantize_int8_per_block")
+               : set_error(FS_ERR_INVALID, "quantize: dtype code must be 0, 1 or 2");
 }
 
 extern "C" int fs_dequantize_i8(const int8_t* values, const float* scale, const int16_t* zero, int64_t outer,
@@ -751,23 +810,62 @@ extern "C" int fs_quantize_pages_i8(const void* x, int x_dtype, int batch, int h
   const int64_t groups = num_pages * heads;
   if (groups > 0x7fffffffLL) return set_error(FS_ERR_INVALID, "quantize_pages: more than 2^31 (page, head) groups");
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  const int ch = vec_chunks(page_size, head_dim);
-  if (is_pow2_chunks(ch) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0) {
-    switch (x_dtype) {
-      case FS_F32: return launch_vec_pages<float>(ch, vec_grid(groups), st, (const float*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
-      case FS_F16: return launch_vec_pages<__half>(ch, vec_grid(groups), st, (const __half*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
-      case FS_BF16: return launch_vec_pages<__hip_bfloat16>(ch, vec_grid(groups), st, (const __hip_bfloat16*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
-      default: return set_error(FS_ERR_INVALID, "quantize_pages: dtype code must be 0, 1 or 2");
-    }
+  const int ch = ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 ? group_chunks(page_size, head_dim) : 0;
+  const bool known = by_dtype(x_dtype, [&](auto tag) {
+    using XT = value_of<decltype(tag)>;
+    const XT* src = (const XT*)x;
+    if (ch == 0)
+      hipLaunchKernelGGL(quantize_pages_kernel<XT>, wave_grid(groups), dim3(256), 0, st, src, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
+    else
+      by_chunks(ch, [&](auto c) {
+        hipLaunchKernelGGL((quantize_pages_vec_kernel<decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
+      });
+  });
+  return known ? check_launch("quantize_pages")
+               : set_error(FS_ERR_INVALID, "quantize_pages: dtype code must be 0, 1 or 2");
+}
+
+extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, int src_tokens, int length, int heads,
+                                  int head_dim, int page_size, int8_t* k_values, float* k_scale, int16_t* k_zero,
+                                  int8_t* v_values, float* v_scale, int16_t* v_zero, int64_t num_pages,
+                                  const int32_t* pages, int n_pages, void* stream) {
+  if (heads <= 0 || head_dim <= 0 || page_size <= 0 || length <= 0 || src_tokens < length || num_pages <= 0)
+    return set_error(FS_ERR_INVALID, "write_prompt: sizes must be positive and length at most src_tokens");
+  if (n_pages != (int)(((int64_t)length + page_size - 1) / page_size))
+    return set_error(FS_ERR_INVALID, "write_prompt: n_pages must equal ceil(length / page_size)");
+  if (!k || !pages || !k_values || !k_scale || !k_zero || (v && (!v_values || !v_scale || !v_zero)))
+    return set_error(FS_ERR_INVALID, "write_prompt: null pointer");
+  if ((int64_t)n_pages * page_size > 0x7fffffffLL || (int64_t)page_size * head_dim > 0x7fffffffLL)
+    return set_error(FS_ERR_INVALID, "write_prompt: sizes past 2^31");
+  for (int i = 0; i < n_pages; ++i)
+    if (pages[i] < 0 || pages[i] >= num_pages) return set_error(FS_ERR_INVALID, "write_prompt: page id out of range");
+  hipStream_t st = (hipStream_t)stream;
+  const uintptr_t src_bits = (uintptr_t)k | (uintptr_t)v, dst_bits = (uintptr_t)k_values | (v ? (uintptr_t)v_values : 0);
+  const int ch = src_bits % 16 == 0 && dst_bits % 8 == 0 ? group_chunks(page_size, head_dim) : 0;
+  const int sides = v ? 2 : 1;
+  if ((int64_t)sides * kPromptPages * heads > 0x7fffffffLL)
+    return set_error(FS_ERR_INVALID, "write_prompt: too many (page, head) groups");
+  PromptPages ids;
+  for (int first = 0; first < n_pages; first += kPromptPages) {
+    const int n = n_pages - first < kPromptPages ? n_pages - first : kPromptPages;
+    for (int i = 0; i < n; ++i) ids.id[i] = pages[first + i];
+    for (int i = n; i < kPromptPages; ++i) ids.id[i] = 0;
+    const int64_t groups = (int64_t)sides * n * heads;
+    const bool known = by_dtype(src_dtype, [&](auto tag) {
+      using XT = value_of<decltype(tag)>;
+      const PromptSource<XT> s{(const XT*)k, (const XT*)v, {k_values, k_scale, k_zero}, {v_values, v_scale, v_zero},
+                               heads, src_tokens, length, head_dim, page_size, first, n};
+      if (ch == 0)
+        hipLaunchKernelGGL(prompt_pages_kernel<XT>, wave_grid(groups), dim3(256), 0, st, s, groups, ids);
+      else
+        by_chunks(ch, [&](auto c) {
+          hipLaunchKernelGGL((prompt_pages_vec_kernel<decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, s, groups, ids);
+        });
+    });
+    if (!known) return set_error(FS_ERR_INVALID, "write_prompt: dtype code must be 0, 1 or 2");
+    if (const int rc = check_launch("write_prompt")) return rc;
   }
-  switch (x_dtype) {
-    case FS_F32: hipLaunchKernelGGL(quantize_pages_kernel<float>, grid, block, 0, st, (const float*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero); break;
-    case FS_F16: hipLaunchKernelGGL(quantize_pages_kernel<__half>, grid, block, 0, st, (const __half*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero); break;
-    case FS_BF16: hipLaunchKernelGGL(quantize_pages_kernel<__hip_bfloat16>, grid, block, 0, st, (const __hip_bfloat16*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero); break;
-    default: return set_error(FS_ERR_INVALID, "quantize_pages: dtype code must be 0, 1 or 2");
-  }
-  return check_launch("quantize_pages");
+  return FS_OK;
 }
 
 extern "C" int fs_update_pages_i8(const int8_t* in_values, const float* in_scale, const int16_t* in_zero,

@@ -8,12 +8,13 @@ maps logical pages to physical ones.
 On GPU every quantized write goes through the HIP page kernels:
 ``fs_quantize_pages_i8`` for ``from_dense`` and ``fs_update_pages_i8`` for
 ``append`` (whole-store requantization, as the reference does) and for the
-allocator's prompt/append writes (only the touched pages).  Host bookkeeping —
+allocator's append writes (only the touched pages), ``fs_write_prompt_i8`` for its prompts.  Host bookkeeping —
 free list, tables, lengths — stays in Python like the reference's.
 """
 
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass
 from typing import Dict, Sequence, Tuple
 
@@ -50,7 +51,7 @@ def _src_for_kernel(x: torch.Tensor) -> torch.Tensor:
 
 
 def _update_pages(store: QuantizedTensor, out: Tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None,
-                  pages: np.ndarray | None, n_pages: int, fresh: np.ndarray | None, row_src: np.ndarray,
+                  pages: np.ndarray | None, n_pages: int, row_src: np.ndarray,
                   src: torch.Tensor, *, heads: int, page: int, dim: int) -> None:
     """One ``fs_update_pages_i8`` call; ``out=None`` updates ``store`` in place."""
 
@@ -70,13 +71,12 @@ def _update_pages(store: QuantizedTensor, out: Tuple[torch.Tensor, torch.Tensor,
     src_t = _src_for_kernel(src)
     rs = torch.from_numpy(np.ascontiguousarray(row_src, dtype=np.int32)).to(dev, non_blocking=False)
     pg = None if pages is None else torch.from_numpy(np.ascontiguousarray(pages, dtype=np.int64)).to(dev)
-    fr = None if fresh is None else torch.from_numpy(np.ascontiguousarray(fresh, dtype=np.uint8)).to(dev)
     _lib.check(lib.fs_update_pages_i8(
         in_values.data_ptr(), in_scale.data_ptr(), in_zero.data_ptr(), in_pages, in_qb,
         out_values.data_ptr(), out_scale.data_ptr(), out_zero.data_ptr(),
-        _lib.ptr(pg), _lib.ptr(fr), n_pages, rs.data_ptr(), src_t.data_ptr(), _lib.dtype_code(src_t.dtype),
+        _lib.ptr(pg), None, n_pages, rs.data_ptr(), src_t.data_ptr(), _lib.dtype_code(src_t.dtype),
         int(src_t.shape[2]), heads, page, dim, _lib.stream_ptr(dev)))
-    # rs/pg/fr/src_t may be freed now: the caching allocator hands their blocks out again
+    # rs/pg/src_t may be freed now: the caching allocator hands their blocks out again
     # only to work ordered after this launch on the same stream.
 
 
@@ -147,19 +147,11 @@ class PagedKVAllocator:
         blocks_needed = (effective_length + self.block_size - 1) // self.block_size
         if len(self._free_blocks) < blocks_needed:
             raise RuntimeError("PagedKVAllocator is out of physical blocks")
-        logical_blocks = [self._allocate_block() for _ in range(blocks_needed)]
+        logical_blocks = self._free_blocks[:blocks_needed]
+        del self._free_blocks[:blocks_needed]
         if blocks_needed:
             if self.device.type == "cuda":
-                row_src = np.full((blocks_needed, self.block_size), -1, dtype=np.int32)
-                for lb in range(blocks_needed):
-                    start = lb * self.block_size
-                    width = max(0, min(self.block_size, effective_length - start))
-                    row_src[lb, :width] = np.arange(start, start + width)
-                pages = np.asarray(logical_blocks, dtype=np.int64)
-                fresh = np.ones(blocks_needed, dtype=np.uint8)
-                for store, src in ((self.k_quant, k), (self.v_quant, v)):
-                    _update_pages(store, None, pages, blocks_needed, fresh, row_src, src,
-                                  heads=self.heads, page=self.block_size, dim=self.head_dim)
+                self._write_prompt(k, v, effective_length, logical_blocks)
             else:
                 for lb, physical_idx in enumerate(logical_blocks):
                     start = lb * self.block_size
@@ -170,6 +162,31 @@ class PagedKVAllocator:
                     vb[:, :, : end - start] = v[:, :, start:end].to(device=self.device, dtype=torch.float32)
                     self._write_quantized_block(physical_idx, kb, vb)
         self._requests[request_id] = _RequestBlocks(logical_blocks=logical_blocks, length=effective_length)
+
+    def _write_prompt(self, k: torch.Tensor, v: torch.Tensor, length: int, pages: list[int]) -> None:
+        """Rows [0, length) of ``k`` and ``v`` into ``pages``: one ``fs_write_prompt_i8`` launch for both
+        (one each when their dtypes differ); the page ids travel with the launch."""
+
+        lib = _lib.require()
+        for store in (self.k_quant, self.v_quant):
+            if not (store.values.is_contiguous() and store.scale.is_contiguous() and store.zero_point.is_contiguous()):
+                raise ValueError("in-place page update needs a contiguous store")
+        ids = array("i", pages)
+
+        def launch(src, store, src2, store2) -> None:
+            _lib.check(lib.fs_write_prompt_i8(
+                src.data_ptr(), _lib.ptr(src2), _lib.dtype_code(src.dtype), int(src.shape[2]), length, self.heads,
+                self.head_dim, self.block_size, store.values.data_ptr(), store.scale.data_ptr(),
+                store.zero_point.data_ptr(), store2.values.data_ptr(), store2.scale.data_ptr(),
+                store2.zero_point.data_ptr(), self.capacity_blocks, ids.buffer_info()[0], len(ids),
+                _lib.stream_ptr(self.device)))
+
+        ks, vs = _src_for_kernel(k), _src_for_kernel(v)
+        if ks.dtype == vs.dtype:
+            launch(ks, self.k_quant, vs, self.v_quant)
+        else:
+            launch(ks, self.k_quant, None, self.k_quant)
+            launch(vs, self.v_quant, None, self.v_quant)
 
     def _plan_append(self, request: _RequestBlocks, tokens: int, touched: Dict[int, list]) -> None:
         """Allocate pages crossed by `tokens` new rows; record (offset, token) per touched page."""
@@ -232,7 +249,7 @@ class PagedKVAllocator:
         page_arr = np.asarray(pages, dtype=np.int64)
         row_src = np.stack(rows)
         for store, src in ((self.k_quant, k_src), (self.v_quant, v_src)):
-            _update_pages(store, None, page_arr, len(pages), None, row_src, src,
+            _update_pages(store, None, page_arr, len(pages), row_src, src,
                           heads=self.heads, page=self.block_size, dim=self.head_dim)
 
     def append_batch(self, request_ids: Sequence[int], k_new: torch.Tensor, v_new: torch.Tensor) -> None:
@@ -594,7 +611,7 @@ class PagedKVCache:
         new_stores = []
         for q, src in ((self.k_quant, k_new), (self.v_quant, v_new)):
             out = _empty_page_store(total, heads, bs, dim, dev)
-            _update_pages(q, out, None, total, None, row_src, src, heads=heads, page=bs, dim=dim)
+            _update_pages(q, out, None, total, row_src, src, heads=heads, page=bs, dim=dim)
             new_stores.append(QuantizedTensor(out[0], out[1], out[2], bs, (total, heads, bs, dim)))
         lengths = lengths + tokens
         return PagedKVCache(

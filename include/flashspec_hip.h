@@ -445,6 +445,17 @@ int fs_update_pages_i8(const int8_t* in_values, const float* in_scale, const int
                        const int32_t* row_src, const void* src, int src_dtype, int src_tokens,
                        int heads, int page_size, int head_dim, void* stream);
 
+/* A prompt's K and V rows into pages of the store (replaces the page writes of reference
+ * paged.py:66-106): rows [0, length) of k and v [heads, src_tokens, head_dim] are quantized page by
+ * page, as fs_update_pages_i8 writes fresh pages (rows past length are zero and take part in the last
+ * page's range), into pages[0 .. n_pages) of both stores.  `pages` is HOST memory, read before the
+ * call returns; n_pages == ceil(length / page_size).  v may be NULL (K alone; its store is unused).
+ * One launch per 896 pages. */
+int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, int src_tokens, int length, int heads,
+                       int head_dim, int page_size, int8_t* k_values, float* k_scale, int16_t* k_zero,
+                       int8_t* v_values, float* v_scale, int16_t* v_zero, int64_t num_pages,
+                       const int32_t* pages, int n_pages, void* stream);
+
 /* One decode step's append, device-resident: for every request b, the token
  * k_new/v_new[b] ([batch, heads, 1, head_dim], dtype src_dtype) goes to position
  * pos = lengths_in[b], i.e. row pos % page_size of physical page block_table[b, pos / page_size];

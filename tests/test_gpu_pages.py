@@ -1,0 +1,152 @@
+"""GPU: K/V written into pages by the register-resident quantizers, bit for bit against the oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import flashspec_amd as fa
+from flashspec_amd import _lib
+from oracle import paged as op
+from oracle import quant as oq
+
+from _helpers import assert_quant_equal, from_qt, np_of, randn
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def announce(msg: str) -> None:
+    print(f"[case] {msg}", flush=True)
+
+
+def shifted(x: torch.Tensor) -> torch.Tensor:
+    """The same values at an address that is no multiple of 16 bytes."""
+
+    base = torch.empty(x.numel() + 1, dtype=x.dtype, device=DEV)
+    base[1:] = x.reshape(-1).to(DEV)
+    return base[1:].reshape(x.shape)
+
+
+# groups of page * D values: 512 multiples (1, 4, 8 chunks), partial chunks (D 80, 96, 112, 24: 2.5,
+# 3, 3.5 and under one), 5 and 7 chunks (run as 6 and 8), over 8 chunks and D no multiple of 8
+# (element-wise); lengths of one token, whole pages and ragged; 898 pages take two launches
+@pytest.mark.parametrize("heads,dim,page,length,dtype", [
+    (3, 32, 16, 1, torch.float16),
+    (4, 128, 16, 301, torch.float16),
+    (2, 256, 16, 32, torch.float32),
+    (5, 80, 16, 83, torch.bfloat16),
+    (2, 96, 16, 47, torch.float32),
+    (2, 112, 16, 65, torch.float16),
+    (3, 24, 16, 50, torch.bfloat16),
+    (2, 160, 16, 33, torch.float16),
+    (2, 224, 16, 40, torch.bfloat16),
+    (2, 80, 32, 70, torch.float16),
+    (2, 256, 32, 70, torch.float16),
+    (2, 36, 16, 35, torch.float16),
+    (1, 8, 16, 897 * 16 + 5, torch.float16),
+])
+def test_prompt_pages_bit_exact(heads, dim, page, length, dtype):
+    announce(f"add_request H{heads} D{dim} page{page} L{length} {dtype}")
+    pages = -(-length // page)
+    alloc = fa.PagedKVAllocator(capacity_blocks=pages + 4, heads=heads, head_dim=dim, block_size=page, device=DEV)
+    ora = op.OracleAllocator(pages + 4, heads, dim, page)
+    for rid, n in ((0, page), (1, page + 1), (2, 1)):
+        k, v = randn((1, heads, n, dim), 10 + rid, dtype), randn((1, heads, n, dim), 20 + rid, dtype)
+        alloc.add_request(rid, k.to(DEV), v.to(DEV))
+        ora.add_request(rid, np_of(k.float()), np_of(v.float()))
+    for a in (alloc, ora):  # the prompt takes the pages in front of request 2 and those behind it
+        a.release_request(1)
+        a.release_request(0)
+    # three rows more than the request keeps
+    k, v = randn((1, heads, length + 3, dim), 1, dtype) * 3.0, randn((1, heads, length + 3, dim), 2, dtype)
+    alloc.add_request(7, k.to(DEV), v.to(DEV), length=length)
+    ora.add_request(7, np_of(k[:, :, :length].float()), np_of(v[:, :, :length].float()))
+    torch.cuda.synchronize()
+    assert_quant_equal(from_qt(alloc.k_quant), ora.k_quant, "k")
+    assert_quant_equal(from_qt(alloc.v_quant), ora.v_quant, "v")
+
+
+def test_prompt_of_two_dtypes_and_unaligned_sources():
+    announce("add_request fp16 K and fp32 V; 2-byte-offset sources")
+    heads, dim, page, length = 2, 128, 16, 39
+    k, v = randn((1, heads, length, dim), 3), randn((1, heads, length, dim), 4, torch.float32)
+    ora = op.OracleAllocator(6, heads, dim, page)
+    ora.add_request(0, np_of(k.float()), np_of(v))
+    ora.add_request(1, np_of(k.float()), np_of(k.float()))
+    alloc = fa.PagedKVAllocator(capacity_blocks=6, heads=heads, head_dim=dim, block_size=page, device=DEV)
+    alloc.add_request(0, k.to(DEV), v.to(DEV))
+    alloc.add_request(1, shifted(k), shifted(k))
+    torch.cuda.synchronize()
+    assert_quant_equal(from_qt(alloc.k_quant), ora.k_quant, "k")
+    assert_quant_equal(from_qt(alloc.v_quant), ora.v_quant, "v")
+
+
+@pytest.mark.parametrize("dim,block,seq,dtype", [
+    (80, 16, 33, torch.float16),
+    (96, 16, 48, torch.bfloat16),
+    (24, 8, 21, torch.float32),
+    (160, 16, 20, torch.float16),
+    (224, 16, 17, torch.float32),
+])
+def test_partial_chunks_bit_exact(dim, block, seq, dtype):
+    """Groups that are no multiple of 512 values, extreme values among them."""
+
+    announce(f"quantize blocks and pages D{dim} block{block} S{seq} {dtype}")
+    x = randn((2, 3, seq, dim), dim + seq, dtype) * 2.0
+    x[0, 0, 1, 1], x[1, 2, seq - 1, dim - 1] = 60000.0, -60000.0
+    x[1] += 100.0  # ranges without zero: a repeated value must not widen them
+    ref = oq.quantize_int8_per_block(np_of(x.float()), block)
+    got = fa.quantize_int8_per_block(x.to(DEV), block)
+    cache = fa.PagedKVCache.from_dense(x.to(DEV), x.to(DEV), block, block_table_pattern="shuffled", layout_seed=1)
+    torch.cuda.synchronize()
+    assert_quant_equal(from_qt(got), ref, "blocks")
+    table = cache.block_table.cpu().numpy()
+    for b in range(2):
+        for i in range(table.shape[1]):
+            assert np.array_equal(np_of(cache.k_quant.values)[table[b, i], :, 0], ref.values[b, :, i])
+            assert np.array_equal(np_of(cache.k_quant.scale)[table[b, i]].reshape(-1).view(np.uint32),
+                                  ref.scale[b, :, i].reshape(-1).view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_infinities_nan_and_scratch_ranges_match_the_general_path(dtype):
+    """Aligned sources take the register-resident kernel, unaligned ones the element-wise kernel."""
+
+    announce(f"extreme values, both quantizers, {dtype}")
+    x = randn((10, 1, 16, 80), 5, dtype)
+    big = torch.finfo(dtype).max
+    x[0, 0, 3, 7] = float("inf")
+    x[1, 0, 3, 7] = float("-inf")
+    x[2, 0, 3, 7], x[2, 0, 4, 8] = float("inf"), float("-inf")
+    x[3, 0, 3, 7] = float("nan")
+    x[4] = float("nan")
+    x[5, 0, 0, 0], x[5, 0, 1, 0] = big, -big  # a range past fp32 in fp32 and bf16
+    x[6] = 0.0
+    x[7] = -0.0
+    x[8] *= torch.finfo(dtype).tiny
+    x[9] = big
+    a, b = fa.quantize_int8_per_block(x.to(DEV), 16), fa.quantize_int8_per_block(shifted(x), 16)
+    torch.cuda.synchronize()
+    assert torch.equal(a.values, b.values)
+    assert torch.equal(a.scale.view(torch.int32), b.scale.view(torch.int32))
+    assert torch.equal(a.zero_point, b.zero_point)
+
+
+def test_prompt_entry_rejects_bad_sizes():
+    lib = _lib.require()
+    ids = (np.zeros(4, dtype=np.int32)).ctypes.data
+    bad = [  # length past the source, page count, head_dim, dtype, null pages
+        (1, 1, 1, 8, 9, 2, 64, 16, 1, 1, 1, 1, 1, 1, 4, ids, 1, None),
+        (1, 1, 1, 8, 8, 2, 64, 16, 1, 1, 1, 1, 1, 1, 4, ids, 2, None),
+        (1, 1, 1, 8, 8, 2, 0, 16, 1, 1, 1, 1, 1, 1, 4, ids, 1, None),
+        (1, 1, 9, 8, 8, 2, 64, 16, 1, 1, 1, 1, 1, 1, 4, ids, 1, None),
+        (1, 1, 1, 8, 8, 2, 64, 16, 1, 1, 1, 1, 1, 1, 4, None, 1, None),
+        (1, 1, 1, 8, 8, 2, 64, 16, 1, 1, 1, 1, 1, 1, 0, ids, 1, None),
+    ]
+    for args in bad:
+        assert lib.fs_write_prompt_i8(*args) == _lib.FS_ERR_INVALID
+    past = np.array([4], dtype=np.int32)
+    assert lib.fs_write_prompt_i8(1, 1, 1, 8, 8, 2, 64, 16, 1, 1, 1, 1, 1, 1, 4, past.ctypes.data, 1,
+                                  None) == _lib.FS_ERR_INVALID
