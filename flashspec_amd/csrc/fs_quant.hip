@@ -94,31 +94,68 @@ __device__ __forceinline__ void quantize_channel_group(const Get& get, int rows,
   }
 }
 
-// Group formats of the element-wise block / page quantizers.
+// Symmetric absmax INT8 over a group of `rows` tokens, one scale per token row:
+// scale = max(absmax / 127, 1e-8), q = clamp(rint(x / scale), -127, 127), zero point 128.
+template <typename Get>
+__device__ __forceinline__ void quantize_token_group(const Get& get, int rows, int D, int8_t* dst, float* scale_out,
+                                                     int16_t* zero_out, int lane) {
+  for (int r = 0; r < rows; ++r) {
+    float am = 0.0f;
+    for (int d = lane; d < D; d += kWave) am = fmaxf(am, fabsf(get(r, d)));
+    am = wave_max(am);
+    const float s = fmaxf(am / 127.0f, 1.0e-8f);
+    for (int d = lane; d < D; d += kWave)
+      dst[(size_t)r * D + d] = (int8_t)(int)fminf(fmaxf(__builtin_rintf(get(r, d) / s), -127.0f), 127.0f);
+    if (lane == 0) {
+      scale_out[r] = s;
+      zero_out[r] = 128;
+    }
+  }
+}
+
+// Group formats of the block / page quantizers.
 enum GroupFormat : int {
   kGfAffine = 0,   // affine INT8, one scale / zero per group
   kGfFp8 = 1,      // FP8 E4M3, one scale per group, zero 0
   kGfChannel = 2,  // affine INT8, one scale / zero per channel of the group
+  kGfToken = 3,    // symmetric INT8, one scale per row of the group, zero 128
 };
+
+// scale / zero entries of one group
+template <int GF>
+__host__ __device__ constexpr int group_params(int rows, int D) {
+  return GF == kGfChannel ? D : (GF == kGfToken ? rows : 1);
+}
 
 template <int GF, typename Get>
 __device__ __forceinline__ void quantize_any_group(const Get& get, int rows, int D, int8_t* dst, float* scale,
                                                    int16_t* zero, int64_t grp, int lane) {
+  scale += (size_t)grp * group_params<GF>(rows, D);
+  if (zero) zero += (size_t)grp * group_params<GF>(rows, D);
   if constexpr (GF == kGfFp8)
-    quantize_group_fp8(get, rows, D, dst, scale + grp, zero ? zero + grp : nullptr, lane);
+    quantize_group_fp8(get, rows, D, dst, scale, zero, lane);
   else if constexpr (GF == kGfChannel)
-    quantize_channel_group(get, rows, D, dst, scale + grp * D, zero + grp * D, lane);
+    quantize_channel_group(get, rows, D, dst, scale, zero, lane);
+  else if constexpr (GF == kGfToken)
+    quantize_token_group(get, rows, D, dst, scale, zero, lane);
   else
-    quantize_group(get, rows, D, dst, scale + grp, zero + grp, lane);
+    quantize_group(get, rows, D, dst, scale, zero, lane);
 }
 
 // ---- vectorized group quantizer --------------------------------------------------------------
-// Same arithmetic as quantize_group, for a group of `rows` contiguous source rows of D values with
-// D % 8 == 0 and n = rows*D <= CH*512: lane l holds values [c*512 + 8l, c*512 + 8l + 8) of every
-// chunk c in registers, read once from HBM with 16-byte loads (non-temporal: the source is read
-// exactly once) and written back as 8-byte packed stores.  Lanes past the group's n values (head
-// dims such as 80, whose groups are no multiple of 512) hold its first eight again, which leaves
-// the extremes as they are, and store nothing.
+// Same arithmetic as the element-wise groups above, for a group of `rows` contiguous source rows of
+// D values with D % 8 == 0, held in registers: read once from HBM with 16-byte loads (non-temporal:
+// the source is read exactly once) and written back as 8-byte packed stores.  Lane l holds, of every
+// chunk c < CH, the 8 values at c * step + 8 l (LaneMap).  With one parameter per group a chunk is
+// 512 values in a row.  With one per channel or row a chunk is as many whole rows as 64 lanes hold,
+// so that a lane keeps its 8 channels in every chunk and a row stays in neighbouring lanes.  Lanes
+// and chunks past the group's n values hold values of the group again (of the same channels), which
+// leaves every extreme as it is, and store nothing.
+//
+// Bound by HBM: 2 bytes read and 1 written per 16-bit value.  The element-wise kernels read every
+// value twice (once for the range) and divided it with the 10-instruction IEEE sequence.  Measured on
+// MI355X, from_dense of bf16 [4, 32, 2039, 128] to shuffled FP8 pages, the whole call: 174 us (2 x 78 us
+// of element-wise kernels) -> 76.8 us.
 
 typedef uint32_t q_u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -182,14 +219,37 @@ struct RawGroup {
   q_u32x4_t w[kWords];
 };
 
+struct LaneMap {
+  int step;   // values per chunk
+  int first;  // the lane's first value in a chunk (n or more: the lane holds none of its own)
+  int alt;    // what it holds where it has none
+  int lpr, rpw;  // row formats: lanes per row, rows per chunk
+  int row, col;  // the lane's row within a chunk and lane within the row
+};
+
+template <int GF>
+__device__ __forceinline__ LaneMap lane_map(int n, int D, int lane) {
+  LaneMap m{512, lane * 8, 0, 0, 0, 0, 0};
+  if constexpr (GF == kGfChannel || GF == kGfToken) {
+    m.lpr = D / 8;
+    m.rpw = kWave / m.lpr;
+    m.row = lane / m.lpr;
+    m.col = lane - m.row * m.lpr;
+    m.step = m.rpw * D;
+    m.first = m.row < m.rpw ? lane * 8 : n;
+    m.alt = m.col * 8;
+  }
+  return m;
+}
+
 // `valid`: the group's values that exist in the source, `n` its values with the zero rows.
 template <int CH, typename XT>
-__device__ __forceinline__ void load_raw(RawGroup<CH, XT>& r, const XT* src, int valid, int n, int lane) {
+__device__ __forceinline__ void load_raw(RawGroup<CH, XT>& r, const XT* src, int valid, int n, const LaneMap& m) {
   constexpr int per = RawGroup<CH, XT>::kWords / CH;  // 16-byte words per chunk
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int at = c * 512 + lane * 8;
-    const int e = at < n ? at : 0;
+    const int at = c * m.step + m.first;
+    const int e = at < n ? at : m.alt;
     const bool ok = e < valid;
 #pragma unroll
     for (int i = 0; i < per; ++i)
@@ -252,6 +312,199 @@ __device__ __forceinline__ void quantize_regs(const float (&x)[CH][8], int8_t* d
   }
 }
 
+// FP8 E4M3 (quantize_group_fp8's op sequence).  The quotient takes its value's sign back: the
+// correction step loses the sign of a zero quotient, and FP8 codes keep it.
+template <int CH, bool RCP>
+__device__ __forceinline__ void store_chunks_fp8(const float (&x)[CH][8], float scale, float rcp, int8_t* dst, int n,
+                                                 int lane) {
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float qd = RCP ? __builtin_copysignf(div_by_scale(x[c][i], scale, rcp), x[c][i]) : x[c][i] / scale;
+      y[i] = fminf(fmaxf(qd, -448.0f), 448.0f);
+    }
+    int w[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      w[j] = __builtin_amdgcn_cvt_pk_fp8_f32(y[4 * j], y[4 * j + 1], 0, false);
+      w[j] = __builtin_amdgcn_cvt_pk_fp8_f32(y[4 * j + 2], y[4 * j + 3], w[j], true);
+    }
+    const int e = c * 512 + lane * 8;
+    if (e < n) *(uint2*)(dst + e) = make_uint2((uint32_t)w[0], (uint32_t)w[1]);
+  }
+}
+
+template <int CH>
+__device__ __forceinline__ void quantize_regs_fp8(const float (&x)[CH][8], int8_t* dst, float* scale_out,
+                                                  int16_t* zero_out, int n, int lane) {
+  float am = 0.0f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(x[c][i]));
+  }
+  am = wave_max_valu(am);
+  const float scale = fmaxf(am / 448.0f, 1.0e-8f);
+  const float rcp = 1.0f / scale;
+  if (__builtin_isfinite(am * rcp))  // wave-uniform, as in quantize_regs
+    store_chunks_fp8<CH, true>(x, scale, rcp, dst, n, lane);
+  else
+    store_chunks_fp8<CH, false>(x, scale, rcp, dst, n, lane);
+  if (lane == 0) {
+    *scale_out = scale;
+    if (zero_out) *zero_out = 0;
+  }
+}
+
+// Per channel (quantize_channel_group's op sequence): each lane reduces its 8 channels over its own
+// rows, then over the lanes that hold the same channels.
+template <int CH, bool RCP>
+__device__ __forceinline__ void store_chunks_channel(const float (&x)[CH][8], const float (&scale)[8],
+                                                     const float (&rcp)[8], const float (&zero)[8], int8_t* dst, int n,
+                                                     const LaneMap& m) {
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    uint32_t w[2] = {0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float qd = RCP ? div_by_scale(x[c][i], scale[i], rcp[i]) : x[c][i] / scale[i];
+      const float qv = fminf(fmaxf(__builtin_rintf(qd + zero[i]), 0.0f), 255.0f);
+      w[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(qv, i % 4, w[i / 4]);
+    }
+    const int e = c * m.step + m.first;
+    if (e < n) *(uint2*)(dst + e) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+  }
+}
+
+template <int CH>
+__device__ __forceinline__ void quantize_regs_channel(const float (&x)[CH][8], int8_t* dst, float* scale_out,
+                                                      int16_t* zero_out, int n, const LaneMap& m) {
+  float mn[8], mx[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    mn[i] = __builtin_huge_valf();
+    mx[i] = -__builtin_huge_valf();
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      mn[i] = fminf(mn[i], x[c][i]);
+      mx[i] = fmaxf(mx[i], x[c][i]);
+    }
+  }
+  if ((m.lpr & (m.lpr - 1)) == 0) {
+    for (int off = m.lpr; off < kWave; off <<= 1) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        mn[i] = fminf(mn[i], __shfl_xor(mn[i], off, kWave));
+        mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], off, kWave));
+      }
+    }
+  } else {
+    float own_mn[8], own_mx[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      own_mn[i] = mn[i];
+      own_mx[i] = mx[i];
+    }
+    for (int r = 0; r < m.rpw; ++r) {  // the lanes of every row in turn
+      const int from = r * m.lpr + m.col;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        mn[i] = fminf(mn[i], __shfl(own_mn[i], from, kWave));
+        mx[i] = fmaxf(mx[i], __shfl(own_mx[i], from, kWave));
+      }
+    }
+  }
+  float scale[8], zero[8], rcp[8];
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    scale[i] = fmaxf((mx[i] - mn[i]) / 255.0f, 1.0e-8f);
+    zero[i] = fminf(fmaxf(__builtin_rintf(-mn[i] / scale[i]), 0.0f), 255.0f);
+    rcp[i] = 1.0f / scale[i];
+    finite = finite && __builtin_isfinite(fmaxf(fabsf(mn[i]), fabsf(mx[i])) * rcp[i]);
+  }
+  if (__all(finite))
+    store_chunks_channel<CH, true>(x, scale, rcp, zero, dst, n, m);
+  else
+    store_chunks_channel<CH, false>(x, scale, rcp, zero, dst, n, m);
+  if (m.row == 0) {
+    float4* so = (float4*)(scale_out + 8 * m.col);
+    so[0] = make_float4(scale[0], scale[1], scale[2], scale[3]);
+    so[1] = make_float4(scale[4], scale[5], scale[6], scale[7]);
+    uint32_t z[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = (uint32_t)(int)zero[2 * i] | ((uint32_t)(int)zero[2 * i + 1] << 16);
+    *(uint4*)(zero_out + 8 * m.col) = make_uint4(z[0], z[1], z[2], z[3]);
+  }
+}
+
+// Symmetric per row (quantize_token_group's op sequence): a row's lanes are neighbours.
+template <int CH, bool RCP>
+__device__ __forceinline__ void store_chunks_token(const float (&x)[CH][8], const float (&scale)[CH],
+                                                   const float (&rcp)[CH], int8_t* dst, int n, const LaneMap& m) {
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    uint32_t w[2] = {0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float qd = RCP ? div_by_scale(x[c][i], scale[c], rcp[c]) : x[c][i] / scale[c];
+      const float qv = fminf(fmaxf(__builtin_rintf(qd), -127.0f), 127.0f);
+      w[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(qv + 128.0f, i % 4, w[i / 4]);  // 1 .. 255: exact
+    }
+    const int e = c * m.step + m.first;
+    if (e < n) *(uint2*)(dst + e) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+  }
+}
+
+template <int CH>
+__device__ __forceinline__ void quantize_regs_token(const float (&x)[CH][8], int8_t* dst, float* scale_out,
+                                                    int16_t* zero_out, int n, const LaneMap& m) {
+  float scale[CH], rcp[CH];
+  bool finite = true;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    float am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(x[c][i]));
+    if ((m.lpr & (m.lpr - 1)) == 0) {
+      for (int off = 1; off < m.lpr; off <<= 1) am = fmaxf(am, __shfl_xor(am, off, kWave));
+    } else {
+      const float own = am;
+      for (int j = 0; j < m.lpr; ++j) am = fmaxf(am, __shfl(own, (m.row < m.rpw ? m.row : 0) * m.lpr + j, kWave));
+    }
+    scale[c] = fmaxf(am / 127.0f, 1.0e-8f);
+    rcp[c] = 1.0f / scale[c];
+    finite = finite && __builtin_isfinite(am * rcp[c]);
+  }
+  if (__all(finite))
+    store_chunks_token<CH, true>(x, scale, rcp, dst, n, m);
+  else
+    store_chunks_token<CH, false>(x, scale, rcp, dst, n, m);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    if (m.col == 0 && c * m.step + m.first < n) {
+      const int r = c * m.rpw + m.row;
+      scale_out[r] = scale[c];
+      zero_out[r] = 128;
+    }
+  }
+}
+
+template <int GF, int CH>
+__device__ __forceinline__ void quantize_any_regs(const float (&x)[CH][8], int8_t* dst, float* scale, int16_t* zero,
+                                                  int n, const LaneMap& m, int lane) {
+  if constexpr (GF == kGfFp8)
+    quantize_regs_fp8<CH>(x, dst, scale, zero, n, lane);
+  else if constexpr (GF == kGfChannel)
+    quantize_regs_channel<CH>(x, dst, scale, zero, n, m);
+  else if constexpr (GF == kGfToken)
+    quantize_regs_token<CH>(x, dst, scale, zero, n, m);
+  else
+    quantize_regs<CH>(x, dst, scale, zero, n, lane);
+}
+
 template <int CH, typename XT>
 __device__ __forceinline__ void unpack_group(const RawGroup<CH, XT>& r, float (&x)[CH][8]) {
   constexpr int per = RawGroup<CH, XT>::kWords / CH;
@@ -271,27 +524,42 @@ struct GroupRef {
 
 // Waves loop over groups grp = wave, wave + waves, ...: the next group's loads are issued before
 // the current group is quantized, so every wave keeps a group's bytes in flight while it computes.
-template <int CH, typename XT, typename Map>
+// Groups of more than 8 chunks leave no registers for a second one: there the other waves cover.
+constexpr int kPipelinedChunks = 8;
+
+template <int GF, int CH, typename XT, typename Map>
 __device__ __forceinline__ void quantize_groups_pipelined(const Map& map, int64_t ngroups, int rows, int D) {
   const int lane = threadIdx.x & (kWave - 1);
   const int n = rows * D;
+  const LaneMap m = lane_map<GF>(n, D, lane);
   const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
   int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   if (grp >= ngroups) return;
+  if constexpr (CH > kPipelinedChunks) {
+    for (; grp < ngroups; grp += waves) {
+      const GroupRef<XT> cur = map(grp);
+      RawGroup<CH, XT> raw;
+      load_raw(raw, cur.src, cur.valid_rows * D, n, m);
+      float x[CH][8];
+      unpack_group(raw, x);
+      quantize_any_regs<GF, CH>(x, cur.dst, cur.scale, cur.zero, n, m, lane);
+    }
+    return;
+  }
   GroupRef<XT> cur = map(grp);
   RawGroup<CH, XT> raw;
-  load_raw(raw, cur.src, cur.valid_rows * D, n, lane);
+  load_raw(raw, cur.src, cur.valid_rows * D, n, m);
   for (;;) {
     const int64_t nxt = grp + waves;
     GroupRef<XT> ref_next{};
     RawGroup<CH, XT> raw_next;
     if (nxt < ngroups) {
       ref_next = map(nxt);
-      load_raw(raw_next, ref_next.src, ref_next.valid_rows * D, n, lane);
+      load_raw(raw_next, ref_next.src, ref_next.valid_rows * D, n, m);
     }
     float x[CH][8];
     unpack_group(raw, x);
-    quantize_regs<CH>(x, cur.dst, cur.scale, cur.zero, n, lane);
+    quantize_any_regs<GF, CH>(x, cur.dst, cur.scale, cur.zero, n, m, lane);
     if (nxt >= ngroups) break;
     grp = nxt;
     cur = ref_next;
@@ -299,12 +567,18 @@ __device__ __forceinline__ void quantize_groups_pipelined(const Map& map, int64_
   }
 }
 
-// 512-value chunks of a group of `rows` rows when the vectorized quantizers apply (rounded up to an
-// instantiated count), else 0.
-static int group_chunks(int64_t rows, int D) {
-  if (D % 8 != 0 || rows * D > 8 * 512) return 0;
-  const int ch = (int)((rows * D + 511) / 512);
-  return ch == 5 ? 6 : (ch == 7 ? 8 : ch);
+// Chunks of a group of `rows` rows when the vectorized quantizers apply (rounded up to an instantiated
+// count), else 0.  `by_row`: the formats whose chunks are whole rows (kGfChannel, kGfToken).
+static int group_chunks(int64_t rows, int D, bool by_row) {
+  if (D % 8 != 0 || rows * D > 16 * 512 || (by_row && D > 512)) return 0;
+  const int64_t per = by_row ? kWave / (D / 8) : 512;
+  const int64_t ch = ((by_row ? rows : rows * D) + per - 1) / per;
+  return ch <= 4 ? (int)ch : (ch <= 6 ? 6 : (ch <= 8 ? 8 : (ch <= 16 ? 16 : 0)));
+}
+
+// Whether scale / zero can be stored 16 bytes at a time (kGfChannel stores them so).
+static bool wide_params(const void* scale, const void* zero) {
+  return ((uintptr_t)scale % 16) == 0 && ((uintptr_t)zero % 16) == 0;
 }
 
 // Chunks of 512 values per group when the vectorized append applies, else 0.
@@ -313,27 +587,29 @@ __host__ __device__ constexpr int vec_chunks(int rows, int D) {
 }
 
 // x [outer, S, D] -> values [outer, nb, bs, D]; groups (o, block), vectorized and pipelined.
-template <int CH, typename XT>
+template <int GF, int CH, typename XT>
 __global__ void __launch_bounds__(256)
 quantize_blocks_vec_kernel(const XT* x, int64_t outer, int S, int D, int bs, int nb, int8_t* values, float* scale,
                            int16_t* zero) {
+  const int per = group_params<GF>(bs, D);
   auto map = [=](int64_t grp) {
     const int64_t o = grp / nb;
     const int blk = (int)(grp - o * nb);
     return GroupRef<XT>{x + ((size_t)o * S + (size_t)blk * bs) * D, min(S - blk * bs, bs), values + (size_t)grp * bs * D,
-                        scale + grp, zero + grp};
+                        scale + (size_t)grp * per, zero ? zero + (size_t)grp * per : nullptr};
   };
-  quantize_groups_pipelined<CH, XT>(map, outer * nb, bs, D);
+  quantize_groups_pipelined<GF, CH, XT>(map, outer * nb, bs, D);
 }
 
 // dense [B, H, S, D] -> page store [P, H, page, D], vectorized and pipelined (see
 // quantize_pages_kernel).
-template <int CH, typename XT>
+template <int GF, int CH, typename XT>
 __global__ void __launch_bounds__(256)
 quantize_pages_vec_kernel(const XT* x, int H, int S, int D, int page, int nbps, const int64_t* page_src, int64_t P,
                           int8_t* values, float* scale, int16_t* zero) {
   // 32-bit index arithmetic (the host keeps P * H < 2^31): a 64-bit division per group sat on
   // the critical path to the next group's loads
+  const int per = group_params<GF>(page, D);
   auto map = [=](int64_t grp) {
     const unsigned j = (unsigned)grp / (unsigned)H;
     const int h = (int)((unsigned)grp - j * (unsigned)H);
@@ -341,9 +617,9 @@ quantize_pages_vec_kernel(const XT* x, int H, int S, int D, int page, int nbps, 
     const unsigned b = o / (unsigned)nbps;
     const int lb = (int)(o - b * (unsigned)nbps);
     return GroupRef<XT>{x + (((size_t)(b * H + h) * S) + (size_t)lb * page) * D, min(S - lb * page, page),
-                        values + (size_t)grp * page * D, scale + grp, zero + grp};
+                        values + (size_t)grp * page * D, scale + (size_t)grp * per, zero ? zero + (size_t)grp * per : nullptr};
   };
-  quantize_groups_pipelined<CH, XT>(map, P * H, page, D);
+  quantize_groups_pipelined<GF, CH, XT>(map, P * H, page, D);
 }
 
 // x [outer, S, D] -> values [outer, nb, bs, D]; group = (o, block); rows past S read as 0.
@@ -471,7 +747,7 @@ template <int CH, typename XT>
 __global__ void __launch_bounds__(256)
 prompt_pages_vec_kernel(const PromptSource<XT> s, int64_t groups, const PromptPages pages) {
   auto map = [&](int64_t grp) { return prompt_group(s, pages, grp); };
-  quantize_groups_pipelined<CH, XT>(map, groups, s.page, s.D);
+  quantize_groups_pipelined<kGfAffine, CH, XT>(map, groups, s.page, s.D);
 }
 
 template <typename XT>
@@ -716,7 +992,8 @@ static void by_chunks(int ch, F&& f) {
     case 3: f(std::integral_constant<int, 3>{}); break;
     case 4: f(std::integral_constant<int, 4>{}); break;
     case 6: f(std::integral_constant<int, 6>{}); break;
-    default: f(std::integral_constant<int, 8>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    default: f(std::integral_constant<int, 16>{}); break;
   }
 }
 
@@ -748,32 +1025,73 @@ static int launch_vec_append(int ch, dim3 grid, hipStream_t st, const XT* k_new,
   return check_launch("append_tokens");
 }
 
+// One launch of the block quantizer of format GF.
+template <int GF>
+static int launch_blocks(const char* what, const void* x, int x_dtype, int64_t outer, int S, int D, int bs,
+                         int8_t* values, float* scale, int16_t* zero, hipStream_t st) {
+  if (outer <= 0 || S <= 0 || D <= 0 || bs <= 0)
+    return set_error(FS_ERR_INVALID, std::string(what) + ": sizes must be positive");
+  if (!x || !values || !scale || (!zero && GF != kGfFp8))
+    return set_error(FS_ERR_INVALID, std::string(what) + ": null pointer");
+  const int nb = (S + bs - 1) / bs;
+  const int64_t groups = outer * nb;
+  if ((groups + 3) / 4 > 0x7fffffffLL) return set_error(FS_ERR_INVALID, std::string(what) + ": too many groups");
+  const bool aligned = ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 &&
+                       (GF != kGfChannel || wide_params(scale, zero));
+  const int ch = aligned ? group_chunks(bs, D, GF == kGfChannel || GF == kGfToken) : 0;
+  const bool known = by_dtype(x_dtype, [&](auto tag) {
+    using XT = value_of<decltype(tag)>;
+    const XT* src = (const XT*)x;
+    if (ch == 0)
+      hipLaunchKernelGGL((quantize_blocks_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
+    else
+      by_chunks(ch, [&](auto c) {
+        hipLaunchKernelGGL((quantize_blocks_vec_kernel<GF, decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
+      });
+  });
+  return known ? check_launch(what) : set_error(FS_ERR_INVALID, std::string(what) + ": dtype code must be 0, 1 or 2");
+}
+
+// One launch of the page quantizer of format GF.
+template <int GF>
+static int launch_pages(const char* what, const void* x, int x_dtype, int batch, int H, int S, int D, int page,
+                        const int64_t* page_src, int64_t P, int8_t* values, float* scale, int16_t* zero,
+                        hipStream_t st) {
+  if (batch <= 0 || H <= 0 || S <= 0 || D <= 0 || page <= 0)
+    return set_error(FS_ERR_INVALID, std::string(what) + ": sizes must be positive");
+  if (!x || !values || !scale || (!zero && GF != kGfFp8))
+    return set_error(FS_ERR_INVALID, std::string(what) + ": null pointer");
+  const int nbps = (S + page - 1) / page;
+  if (P != (int64_t)batch * nbps)
+    return set_error(FS_ERR_INVALID, std::string(what) + ": num_pages must equal batch * ceil(seq_len / page)");
+  const int64_t groups = P * H;
+  const bool counted = groups <= 0x7fffffffLL;  // the vectorized kernel's index arithmetic is 32-bit
+  if (!counted && GF == kGfAffine)
+    return set_error(FS_ERR_INVALID, std::string(what) + ": more than 2^31 (page, head) groups");
+  const bool aligned = counted && ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 &&
+                       (GF != kGfChannel || wide_params(scale, zero));
+  const int ch = aligned ? group_chunks(page, D, GF == kGfChannel || GF == kGfToken) : 0;
+  const bool known = by_dtype(x_dtype, [&](auto tag) {
+    using XT = value_of<decltype(tag)>;
+    const XT* src = (const XT*)x;
+    if (ch == 0)
+      hipLaunchKernelGGL((quantize_pages_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, src, H, S, D, page, nbps, page_src, P, values, scale, zero);
+    else
+      by_chunks(ch, [&](auto c) {
+        hipLaunchKernelGGL((quantize_pages_vec_kernel<GF, decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, H, S, D, page, nbps, page_src, P, values, scale, zero);
+      });
+  });
+  return known ? check_launch(what) : set_error(FS_ERR_INVALID, std::string(what) + ": dtype code must be 0, 1 or 2");
+}
+
 }  // namespace fs
 
 using namespace fs;
 
 extern "C" int fs_quantize_i8(const void* x, int x_dtype, int64_t outer, int seq_len, int head_dim, int block_size,
                               int8_t* values, float* scale, int16_t* zero, void* stream) {
-  if (outer <= 0 || seq_len <= 0 || head_dim <= 0 || block_size <= 0)
-    return set_error(FS_ERR_INVALID, "quantize: sizes must be positive");
-  if (!x || !values || !scale || !zero) return set_error(FS_ERR_INVALID, "quantize: null pointer");
-  const int nb = (seq_len + block_size - 1) / block_size;
-  const int64_t groups = outer * nb;
-  if ((groups + 3) / 4 > 0x7fffffffLL) return set_error(FS_ERR_INVALID, "quantize: too many groups");
-  hipStream_t st = (hipStream_t)stream;
-  const int ch = ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 ? group_chunks(block_size, head_dim) : 0;
-  const bool known = by_dtype(x_dtype, [&](auto tag) {
-    using XT = value_of<decltype(tag)>;
-    const XT* src = (const XT*)x;
-    if (ch == 0)
-      hipLaunchKernelGGL(quantize_blocks_kernel<XT>, wave_grid(groups), dim3(256), 0, st, src, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
-    else
-      by_chunks(ch, [&](auto c) {
-        hipLaunchKernelGGL((quantize_blocks_vec_kernel<decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, outer, seq_len, head_dim, block_size, nb, values, scale, zero);
-      });
-  });
-  return known ? check_launch("quantize_int8_per_block")
-               : set_error(FS_ERR_INVALID, "quantize: dtype code must be 0, 1 or 2");
+  return launch_blocks<kGfAffine>("quantize", x, x_dtype, outer, seq_len, head_dim, block_size, values, scale, zero,
+                                  (hipStream_t)stream);
 }
 
 extern "C" int fs_dequantize_i8(const int8_t* values, const float* scale, const int16_t* zero, int64_t outer,
@@ -801,28 +1119,8 @@ extern "C" int fs_dequantize_i8(const int8_t* values, const float* scale, const 
 extern "C" int fs_quantize_pages_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
                                     int page_size, const int64_t* page_src, int64_t num_pages, int8_t* values,
                                     float* scale, int16_t* zero, void* stream) {
-  if (batch <= 0 || heads <= 0 || seq_len <= 0 || head_dim <= 0 || page_size <= 0)
-    return set_error(FS_ERR_INVALID, "quantize_pages: sizes must be positive");
-  if (!x || !values || !scale || !zero) return set_error(FS_ERR_INVALID, "quantize_pages: null pointer");
-  const int nbps = (seq_len + page_size - 1) / page_size;
-  if (num_pages != (int64_t)batch * nbps)
-    return set_error(FS_ERR_INVALID, "quantize_pages: num_pages must equal batch * ceil(seq_len / page)");
-  const int64_t groups = num_pages * heads;
-  if (groups > 0x7fffffffLL) return set_error(FS_ERR_INVALID, "quantize_pages: more than 2^31 (page, head) groups");
-  hipStream_t st = (hipStream_t)stream;
-  const int ch = ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 ? group_chunks(page_size, head_dim) : 0;
-  const bool known = by_dtype(x_dtype, [&](auto tag) {
-    using XT = value_of<decltype(tag)>;
-    const XT* src = (const XT*)x;
-    if (ch == 0)
-      hipLaunchKernelGGL(quantize_pages_kernel<XT>, wave_grid(groups), dim3(256), 0, st, src, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
-    else
-      by_chunks(ch, [&](auto c) {
-        hipLaunchKernelGGL((quantize_pages_vec_kernel<decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero);
-      });
-  });
-  return known ? check_launch("quantize_pages")
-               : set_error(FS_ERR_INVALID, "quantize_pages: dtype code must be 0, 1 or 2");
+  return launch_pages<kGfAffine>("quantize_pages", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
+                                 num_pages, values, scale, zero, (hipStream_t)stream);
 }
 
 extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, int src_tokens, int length, int heads,
@@ -841,7 +1139,7 @@ extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, i
     if (pages[i] < 0 || pages[i] >= num_pages) return set_error(FS_ERR_INVALID, "write_prompt: page id out of range");
   hipStream_t st = (hipStream_t)stream;
   const uintptr_t src_bits = (uintptr_t)k | (uintptr_t)v, dst_bits = (uintptr_t)k_values | (v ? (uintptr_t)v_values : 0);
-  const int ch = src_bits % 16 == 0 && dst_bits % 8 == 0 ? group_chunks(page_size, head_dim) : 0;
+  const int ch = src_bits % 16 == 0 && dst_bits % 8 == 0 ? group_chunks(page_size, head_dim, false) : 0;
   const int sides = v ? 2 : 1;
   if ((int64_t)sides * kPromptPages * heads > 0x7fffffffLL)
     return set_error(FS_ERR_INVALID, "write_prompt: too many (page, head) groups");
@@ -982,44 +1280,15 @@ extern "C" int fs_quantize_sym_i8(const void* x, int x_dtype, int64_t rows, int 
 
 extern "C" int fs_quantize_fp8(const void* x, int x_dtype, int64_t outer, int seq_len, int head_dim, int block_size,
                                uint8_t* values, float* scale, int16_t* zero, void* stream) {
-  if (outer <= 0 || seq_len <= 0 || head_dim <= 0 || block_size <= 0)
-    return set_error(FS_ERR_INVALID, "quantize_fp8: sizes must be positive");
-  if (!x || !values || !scale) return set_error(FS_ERR_INVALID, "quantize_fp8: null pointer");
-  const int nb = (seq_len + block_size - 1) / block_size;
-  const int64_t groups = outer * nb;
-  if ((groups + 3) / 4 > 0x7fffffffLL) return set_error(FS_ERR_INVALID, "quantize_fp8: too many groups");
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  int8_t* v = (int8_t*)values;
-  switch (x_dtype) {
-    case FS_F32: hipLaunchKernelGGL((quantize_blocks_kernel<float, kGfFp8>), grid, block, 0, st, (const float*)x, outer, seq_len, head_dim, block_size, nb, v, scale, zero); break;
-    case FS_F16: hipLaunchKernelGGL((quantize_blocks_kernel<__half, kGfFp8>), grid, block, 0, st, (const __half*)x, outer, seq_len, head_dim, block_size, nb, v, scale, zero); break;
-    case FS_BF16: hipLaunchKernelGGL((quantize_blocks_kernel<__hip_bfloat16, kGfFp8>), grid, block, 0, st, (const __hip_bfloat16*)x, outer, seq_len, head_dim, block_size, nb, v, scale, zero); break;
-    default: return set_error(FS_ERR_INVALID, "quantize_fp8: dtype code must be 0, 1 or 2");
-  }
-  return check_launch("quantize_fp8_per_block");
+  return launch_blocks<kGfFp8>("quantize_fp8", x, x_dtype, outer, seq_len, head_dim, block_size, (int8_t*)values, scale,
+                               zero, (hipStream_t)stream);
 }
 
 extern "C" int fs_quantize_pages_fp8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
                                      int page_size, const int64_t* page_src, int64_t num_pages, uint8_t* values,
                                      float* scale, int16_t* zero, void* stream) {
-  if (batch <= 0 || heads <= 0 || seq_len <= 0 || head_dim <= 0 || page_size <= 0)
-    return set_error(FS_ERR_INVALID, "quantize_pages_fp8: sizes must be positive");
-  if (!x || !values || !scale) return set_error(FS_ERR_INVALID, "quantize_pages_fp8: null pointer");
-  const int nbps = (seq_len + page_size - 1) / page_size;
-  if (num_pages != (int64_t)batch * nbps)
-    return set_error(FS_ERR_INVALID, "quantize_pages_fp8: num_pages must equal batch * ceil(seq_len / page)");
-  const int64_t groups = num_pages * heads;
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  int8_t* v = (int8_t*)values;
-  switch (x_dtype) {
-    case FS_F32: hipLaunchKernelGGL((quantize_pages_kernel<float, kGfFp8>), grid, block, 0, st, (const float*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, v, scale, zero); break;
-    case FS_F16: hipLaunchKernelGGL((quantize_pages_kernel<__half, kGfFp8>), grid, block, 0, st, (const __half*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, v, scale, zero); break;
-    case FS_BF16: hipLaunchKernelGGL((quantize_pages_kernel<__hip_bfloat16, kGfFp8>), grid, block, 0, st, (const __hip_bfloat16*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, v, scale, zero); break;
-    default: return set_error(FS_ERR_INVALID, "quantize_pages_fp8: dtype code must be 0, 1 or 2");
-  }
-  return check_launch("quantize_pages_fp8");
+  return launch_pages<kGfFp8>("quantize_pages_fp8", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
+                              num_pages, (int8_t*)values, scale, zero, (hipStream_t)stream);
 }
 
 extern "C" int fs_dequantize_fp8(const uint8_t* values, const float* scale, int64_t outer, int n_blocks,
@@ -1045,40 +1314,20 @@ extern "C" int fs_dequantize_fp8(const uint8_t* values, const float* scale, int6
 
 extern "C" int fs_quantize_i8_channel(const void* x, int x_dtype, int64_t outer, int seq_len, int head_dim,
                                       int block_size, int8_t* values, float* scale, int16_t* zero, void* stream) {
-  if (outer <= 0 || seq_len <= 0 || head_dim <= 0 || block_size <= 0)
-    return set_error(FS_ERR_INVALID, "quantize_channel: sizes must be positive");
-  if (!x || !values || !scale || !zero) return set_error(FS_ERR_INVALID, "quantize_channel: null pointer");
-  const int nb = (seq_len + block_size - 1) / block_size;
-  const int64_t groups = outer * nb;
-  if ((groups + 3) / 4 > 0x7fffffffLL) return set_error(FS_ERR_INVALID, "quantize_channel: too many groups");
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  switch (x_dtype) {
-    case FS_F32: hipLaunchKernelGGL((quantize_blocks_kernel<float, kGfChannel>), grid, block, 0, st, (const float*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero); break;
-    case FS_F16: hipLaunchKernelGGL((quantize_blocks_kernel<__half, kGfChannel>), grid, block, 0, st, (const __half*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero); break;
-    case FS_BF16: hipLaunchKernelGGL((quantize_blocks_kernel<__hip_bfloat16, kGfChannel>), grid, block, 0, st, (const __hip_bfloat16*)x, outer, seq_len, head_dim, block_size, nb, values, scale, zero); break;
-    default: return set_error(FS_ERR_INVALID, "quantize_channel: dtype code must be 0, 1 or 2");
-  }
-  return check_launch("quantize_int8_per_channel");
+  return launch_blocks<kGfChannel>("quantize_channel", x, x_dtype, outer, seq_len, head_dim, block_size, values, scale,
+                                   zero, (hipStream_t)stream);
 }
 
 extern "C" int fs_quantize_pages_i8_channel(const void* x, int x_dtype, int batch, int heads, int seq_len,
                                             int head_dim, int page_size, const int64_t* page_src, int64_t num_pages,
                                             int8_t* values, float* scale, int16_t* zero, void* stream) {
-  if (batch <= 0 || heads <= 0 || seq_len <= 0 || head_dim <= 0 || page_size <= 0)
-    return set_error(FS_ERR_INVALID, "quantize_pages_channel: sizes must be positive");
-  if (!x || !values || !scale || !zero) return set_error(FS_ERR_INVALID, "quantize_pages_channel: null pointer");
-  const int nbps = (seq_len + page_size - 1) / page_size;
-  if (num_pages != (int64_t)batch * nbps)
-    return set_error(FS_ERR_INVALID, "quantize_pages_channel: num_pages must equal batch * ceil(seq_len / page)");
-  const int64_t groups = num_pages * heads;
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  switch (x_dtype) {
-    case FS_F32: hipLaunchKernelGGL((quantize_pages_kernel<float, kGfChannel>), grid, block, 0, st, (const float*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero); break;
-    case FS_F16: hipLaunchKernelGGL((quantize_pages_kernel<__half, kGfChannel>), grid, block, 0, st, (const __half*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero); break;
-    case FS_BF16: hipLaunchKernelGGL((quantize_pages_kernel<__hip_bfloat16, kGfChannel>), grid, block, 0, st, (const __hip_bfloat16*)x, heads, seq_len, head_dim, page_size, nbps, page_src, num_pages, values, scale, zero); break;
-    default: return set_error(FS_ERR_INVALID, "quantize_pages_channel: dtype code must be 0, 1 or 2");
-  }
-  return check_launch("quantize_pages_channel");
+  return launch_pages<kGfChannel>("quantize_pages_channel", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
+                                  num_pages, values, scale, zero, (hipStream_t)stream);
+}
+
+extern "C" int fs_quantize_pages_sym_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
+                                        int page_size, const int64_t* page_src, int64_t num_pages, int8_t* values,
+                                        float* scale, int16_t* zero, void* stream) {
+  return launch_pages<kGfToken>("quantize_pages_symmetric", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
+                                num_pages, values, scale, zero, (hipStream_t)stream);
 }

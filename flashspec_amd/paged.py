@@ -36,11 +36,14 @@ def _normalize_device(device: torch.device | str) -> torch.device:
     return dev
 
 
-def _empty_page_store(pages: int, heads: int, page: int, dim: int, device: torch.device, per_channel: bool = False):
-    values = torch.empty((pages, heads, 1, page, dim), dtype=torch.int8, device=device)
-    params = dim if per_channel else 1
-    scale = torch.empty((pages, heads, 1, 1, params), dtype=torch.float32, device=device)
-    zero = torch.empty((pages, heads, 1, 1, params), dtype=torch.int16, device=device)
+def _empty_page_store(pages: int, heads: int, page: int, dim: int, device: torch.device,
+                      kv_format: str = "affine_block"):
+    blocks, rows = (page, 1) if kv_format == "symmetric_token" else (1, page)
+    params = dim if kv_format == "affine_channel" else 1
+    values = torch.empty((pages, heads, blocks, rows, dim), device=device,
+                         dtype=FP8_DTYPE if kv_format == "fp8_block" else torch.int8)
+    scale = torch.empty((pages, heads, blocks, 1, params), dtype=torch.float32, device=device)
+    zero = torch.empty((pages, heads, blocks, 1, params), dtype=torch.int16, device=device)
     return values, scale, zero
 
 
@@ -478,29 +481,17 @@ class PagedKVCache:
             if bool((effective_lengths < 0).any().item()) or bool((effective_lengths > seq_len).any().item()):
                 raise ValueError("lengths must lie in [0, seq_len]")
 
-        if kv_format == "symmetric_token":
-            k_quant = quantize_int8_symmetric_per_token(cls._physical_pages(k, block_size, perm))
-            v_quant = quantize_int8_symmetric_per_token(cls._physical_pages(v, block_size, perm))
-        elif kv_format == "affine_channel":
-            if k.device.type == "cuda":
-                k_quant = cls._quantize_pages(k, block_size, perm, total, per_channel=True)
-                v_quant = cls._quantize_pages(v, block_size, perm, total, per_channel=True)
-            else:
-                k_quant = quantize_int8_per_channel(cls._physical_pages(k, block_size, perm), block_size=block_size)
-                v_quant = quantize_int8_per_channel(cls._physical_pages(v, block_size, perm), block_size=block_size)
-        elif kv_format == "fp8_block":
-            if k.device.type == "cuda":
-                k_quant = cls._quantize_pages(k, block_size, perm, total, fp8=True)
-                v_quant = cls._quantize_pages(v, block_size, perm, total, fp8=True)
-            else:
-                k_quant = quantize_fp8_per_block(cls._physical_pages(k, block_size, perm), block_size=block_size)
-                v_quant = quantize_fp8_per_block(cls._physical_pages(v, block_size, perm), block_size=block_size)
-        elif k.device.type == "cuda":
-            k_quant = cls._quantize_pages(k, block_size, perm, total)
-            v_quant = cls._quantize_pages(v, block_size, perm, total)
+        if k.device.type == "cuda":
+            k_quant = cls._quantize_pages(k, block_size, perm, total, kv_format)
+            v_quant = cls._quantize_pages(v, block_size, perm, total, kv_format)
         else:
-            k_quant = quantize_int8_per_block(cls._physical_pages(k, block_size, perm), block_size=block_size)
-            v_quant = quantize_int8_per_block(cls._physical_pages(v, block_size, perm), block_size=block_size)
+            k_pages, v_pages = cls._physical_pages(k, block_size, perm), cls._physical_pages(v, block_size, perm)
+            if kv_format == "symmetric_token":
+                k_quant, v_quant = map(quantize_int8_symmetric_per_token, (k_pages, v_pages))
+            else:
+                quantize = {"affine_block": quantize_int8_per_block, "fp8_block": quantize_fp8_per_block,
+                            "affine_channel": quantize_int8_per_channel}[kv_format]
+                k_quant, v_quant = quantize(k_pages, block_size=block_size), quantize(v_pages, block_size=block_size)
         return cls(k_quant=k_quant, v_quant=v_quant, block_table=block_table, lengths=effective_lengths,
                    block_size=block_size, max_seq_len=seq_len)
 
@@ -516,25 +507,21 @@ class PagedKVCache:
 
     @staticmethod
     def _quantize_pages(x: torch.Tensor, block_size: int, perm: torch.Tensor | None, total: int,
-                        fp8: bool = False, per_channel: bool = False) -> QuantizedTensor:
+                        kv_format: str) -> QuantizedTensor:
         lib = _lib.require()
         batch, heads, seq_len, head_dim = (int(s) for s in x.shape)
         src = _src_for_kernel(x.detach())
-        values, scale, zero = _empty_page_store(total, heads, block_size, head_dim, x.device, per_channel)
-        if fp8:
-            values = values.view(FP8_DTYPE)
+        values, scale, zero = _empty_page_store(total, heads, block_size, head_dim, x.device, kv_format)
         page_src = None if perm is None else perm.to(torch.int64).contiguous()
-        if fp8:
-            quantize_pages = lib.fs_quantize_pages_fp8
-        elif per_channel:
-            quantize_pages = lib.fs_quantize_pages_i8_channel
-        else:
-            quantize_pages = lib.fs_quantize_pages_i8
+        quantize_pages = {"affine_block": lib.fs_quantize_pages_i8, "fp8_block": lib.fs_quantize_pages_fp8,
+                          "affine_channel": lib.fs_quantize_pages_i8_channel,
+                          "symmetric_token": lib.fs_quantize_pages_sym_i8}[kv_format]
         _lib.check(quantize_pages(
             src.data_ptr(), _lib.dtype_code(src.dtype), batch, heads, seq_len, head_dim, block_size,
             _lib.ptr(page_src), total, values.data_ptr(), scale.data_ptr(), zero.data_ptr(),
             _lib.stream_ptr(x.device)))
-        return QuantizedTensor(values, scale, zero, block_size, (total, heads, block_size, head_dim))
+        return QuantizedTensor(values, scale, zero, 1 if kv_format == "symmetric_token" else block_size,
+                               (total, heads, block_size, head_dim))
 
     def to_dense(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """Dequantize the store and gather ``[batch, heads, max_seq_len, dim]`` (paged.py:421-461)."""

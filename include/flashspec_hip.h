@@ -329,6 +329,12 @@ int fs_quantize_i8(const void* x, int x_dtype, int64_t outer, int seq_len, int h
  */
 int fs_quantize_sym_i8(const void* x, int x_dtype, int64_t rows, int head_dim,
                        int8_t* values, float* scale, int16_t* zero, void* stream);
+/* The same quantizer over the pages of dense [batch, heads, seq_len, head_dim] values, placed as
+ * fs_quantize_pages_i8 places them: values [num_pages, heads, page_size, head_dim], scale / zero
+ * [num_pages, heads, page_size]; rows past seq_len are zero. */
+int fs_quantize_pages_sym_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
+                             int page_size, const int64_t* page_src, int64_t num_pages,
+                             int8_t* values, float* scale, int16_t* zero, void* stream);
 
 /*
  * FP8 E4M3 (OCP "e4m3fn") KV format: per block of block_size tokens x head_dim (zero-padded

@@ -110,12 +110,10 @@ def test_partial_chunks_bit_exact(dim, block, seq, dtype):
                                   ref.scale[b, :, i].reshape(-1).view(np.uint32))
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-def test_infinities_nan_and_scratch_ranges_match_the_general_path(dtype):
-    """Aligned sources take the register-resident kernel, unaligned ones the element-wise kernel."""
+def extreme(dtype: torch.dtype, dim: int) -> torch.Tensor:
+    """Blocks of 16 rows with infinities, NaN, both zeros, the type's largest and tiny values."""
 
-    announce(f"extreme values, both quantizers, {dtype}")
-    x = randn((10, 1, 16, 80), 5, dtype)
+    x = randn((10, 1, 16, dim), 5, dtype)
     big = torch.finfo(dtype).max
     x[0, 0, 3, 7] = float("inf")
     x[1, 0, 3, 7] = float("-inf")
@@ -127,6 +125,85 @@ def test_infinities_nan_and_scratch_ranges_match_the_general_path(dtype):
     x[7] = -0.0
     x[8] *= torch.finfo(dtype).tiny
     x[9] = big
+    return x
+
+
+def assert_same_store(a: fa.QuantizedTensor, b: fa.QuantizedTensor, what: str) -> None:
+    assert a.block_size == b.block_size and a.original_shape == b.original_shape and a.values.dtype == b.values.dtype
+    assert a.values.shape == b.values.shape and a.scale.shape == b.scale.shape, what
+    assert torch.equal(a.values.cpu().view(torch.uint8), b.values.cpu().view(torch.uint8)), what
+    assert torch.equal(a.scale.cpu().view(torch.int32), b.scale.cpu().view(torch.int32)), what
+    assert torch.equal(a.zero_point.cpu(), b.zero_point.cpu()), what
+
+
+FORMATS = ["affine_block", "fp8_block", "affine_channel", "symmetric_token"]
+
+
+# chunks of 512 values (block, FP8) or of whole rows (channel, token): 1, 2, 3 (partial), 4, 6, 8 and
+# 16 chunks, rows of 1, 2, 4, 8, 10, 12, 16, 28 and 32 lanes, head dims and groups that take the
+# element-wise kernel (36, 528; 64-row pages of 256 dims), a last page of one row
+@pytest.mark.parametrize("kv_format", FORMATS)
+@pytest.mark.parametrize("dim,page,seq,dtype", [
+    (8, 16, 17, torch.float16),
+    (16, 8, 30, torch.float32),
+    (32, 16, 64, torch.bfloat16),
+    (64, 16, 49, torch.float16),
+    (80, 16, 33, torch.bfloat16),
+    (96, 32, 70, torch.float16),
+    (128, 16, 301, torch.bfloat16),
+    (128, 64, 130, torch.float16),
+    (224, 16, 40, torch.float16),
+    (256, 16, 48, torch.float32),
+    (256, 32, 65, torch.bfloat16),
+    (256, 64, 70, torch.float16),
+    (36, 16, 35, torch.float16),
+    (528, 4, 9, torch.float32),
+])
+def test_build_matches_the_portable_path_bit_exact(kv_format, dim, page, seq, dtype):
+    announce(f"from_dense {kv_format} D{dim} page{page} S{seq} {dtype}")
+    k, v = randn((3, 2, seq, dim), 1, dtype) * 2.0, randn((3, 2, seq, dim), 2, dtype) + 3.0
+    ref = fa.PagedKVCache.from_dense(k, v, page, block_table_pattern="interleaved", kv_format=kv_format)
+    # K aligned, V at an address that takes the element-wise kernel
+    got = fa.PagedKVCache.from_dense(k.to(DEV), shifted(v), page, block_table_pattern="interleaved",
+                                     kv_format=kv_format)
+    both = fa.PagedKVCache.from_dense(k.to(DEV), v.to(DEV), page, block_table_pattern="interleaved",
+                                      kv_format=kv_format)
+    torch.cuda.synchronize()
+    for cache in (got, both):
+        assert torch.equal(cache.block_table.cpu(), ref.block_table)
+        assert_same_store(cache.k_quant, ref.k_quant, "k")
+        assert_same_store(cache.v_quant, ref.v_quant, "v")
+
+
+@pytest.mark.parametrize("kv_format", FORMATS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [80, 128])
+def test_extreme_values_match_the_general_path_in_every_format(kv_format, dtype, dim):
+    announce(f"extreme values, both page quantizers, {kv_format} {dtype} D{dim}")
+    x = extreme(dtype, dim)
+    a = fa.PagedKVCache.from_dense(x.to(DEV), x.to(DEV), 16, kv_format=kv_format)
+    b = fa.PagedKVCache.from_dense(shifted(x), shifted(x), 16, kv_format=kv_format)
+    torch.cuda.synchronize()
+    assert_same_store(a.k_quant, b.k_quant, "aligned against unaligned")
+
+
+@pytest.mark.parametrize("quantize", [fa.quantize_fp8_per_block, fa.quantize_int8_per_channel])
+@pytest.mark.parametrize("dim,block,seq,dtype", [(80, 16, 33, torch.float16), (128, 16, 300, torch.bfloat16),
+                                                 (256, 32, 40, torch.float32), (64, 8, 21, torch.float16)])
+def test_block_formats_match_the_portable_path_bit_exact(quantize, dim, block, seq, dtype):
+    announce(f"{quantize.__name__} D{dim} block{block} S{seq} {dtype}")
+    x = randn((2, 3, seq, dim), 4, dtype) * 2.0
+    got, ref = quantize(x.to(DEV), block), quantize(x, block)
+    torch.cuda.synchronize()
+    assert_same_store(got, ref, "blocks")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_infinities_nan_and_scratch_ranges_match_the_general_path(dtype):
+    """Aligned sources take the register-resident kernel, unaligned ones the element-wise kernel."""
+
+    announce(f"extreme values, both quantizers, {dtype}")
+    x = extreme(dtype, 80)
     a, b = fa.quantize_int8_per_block(x.to(DEV), 16), fa.quantize_int8_per_block(shifted(x), 16)
     torch.cuda.synchronize()
     assert torch.equal(a.values, b.values)
