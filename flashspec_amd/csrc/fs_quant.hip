@@ -163,6 +163,11 @@ __device__ __forceinline__ q_u32x4_t nt_load16(const void* p) {
   return __builtin_nontemporal_load((const q_u32x4_t*)p);
 }
 
+__device__ __forceinline__ void nt_store8(int8_t* p, uint32_t a, uint32_t b) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(u32x2{a, b}, (u32x2*)p);
+}
+
 __device__ __forceinline__ void load8(const float* p, float* f) {
   const q_u32x4_t a = nt_load16(p), b = nt_load16(p + 4);
 #pragma unroll
@@ -191,6 +196,15 @@ __device__ __forceinline__ void load8(const __hip_bfloat16* p, float* f) {
 }
 
 
+// Chunks that a group running as CH chunks surely fills (group_chunks rounds 5, 7 and 9 to 15 up).
+constexpr int sure_chunks(int CH) { return CH <= 4 ? CH - 1 : (CH == 6 ? 4 : (CH == 8 ? 6 : 8)); }
+
+// Whether the lane has values of its own in chunk c, at e.
+template <int GF, int CH>
+__device__ __forceinline__ bool has_values(int c, int e, int n) {
+  return (GF != kGfChannel && GF != kGfToken && c < sure_chunks(CH)) || e < n;
+}
+
 // Quantize CH chunks of 8 values held by this lane and store them as packed bytes.
 template <int CH, bool RCP>
 __device__ __forceinline__ void store_chunks(const float (&x)[CH][8], float scale, float rcp, float zero,
@@ -207,7 +221,7 @@ __device__ __forceinline__ void store_chunks(const float (&x)[CH][8], float scal
     }
     // stored as q - 128: flip the top bit of every byte
     const int e = c * 512 + lane * 8;
-    if (e < n) *(uint2*)(dst + e) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+    if (has_values<kGfAffine, CH>(c, e, n)) nt_store8(dst + e, w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
   }
 }
 
@@ -243,13 +257,13 @@ __device__ __forceinline__ LaneMap lane_map(int n, int D, int lane) {
 }
 
 // `valid`: the group's values that exist in the source, `n` its values with the zero rows.
-template <int CH, typename XT>
+template <int GF, int CH, typename XT>
 __device__ __forceinline__ void load_raw(RawGroup<CH, XT>& r, const XT* src, int valid, int n, const LaneMap& m) {
   constexpr int per = RawGroup<CH, XT>::kWords / CH;  // 16-byte words per chunk
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     const int at = c * m.step + m.first;
-    const int e = at < n ? at : m.alt;
+    const int e = has_values<GF, CH>(c, at, n) ? at : m.alt;
     const bool ok = e < valid;
 #pragma unroll
     for (int i = 0; i < per; ++i)
@@ -332,7 +346,7 @@ __device__ __forceinline__ void store_chunks_fp8(const float (&x)[CH][8], float 
       w[j] = __builtin_amdgcn_cvt_pk_fp8_f32(y[4 * j + 2], y[4 * j + 3], w[j], true);
     }
     const int e = c * 512 + lane * 8;
-    if (e < n) *(uint2*)(dst + e) = make_uint2((uint32_t)w[0], (uint32_t)w[1]);
+    if (has_values<kGfFp8, CH>(c, e, n)) *(uint2*)(dst + e) = make_uint2((uint32_t)w[0], (uint32_t)w[1]);
   }
 }
 
@@ -374,7 +388,7 @@ __device__ __forceinline__ void store_chunks_channel(const float (&x)[CH][8], co
       w[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(qv, i % 4, w[i / 4]);
     }
     const int e = c * m.step + m.first;
-    if (e < n) *(uint2*)(dst + e) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+    if (e < n) nt_store8(dst + e, w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
   }
 }
 
@@ -454,7 +468,7 @@ __device__ __forceinline__ void store_chunks_token(const float (&x)[CH][8], cons
       w[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(qv + 128.0f, i % 4, w[i / 4]);  // 1 .. 255: exact
     }
     const int e = c * m.step + m.first;
-    if (e < n) *(uint2*)(dst + e) = make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+    if (e < n) nt_store8(dst + e, w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
   }
 }
 
@@ -522,49 +536,25 @@ struct GroupRef {
   int16_t* zero;
 };
 
-// Waves loop over groups grp = wave, wave + waves, ...: the next group's loads are issued before
-// the current group is quantized, so every wave keeps a group's bytes in flight while it computes.
-// Groups of more than 8 chunks leave no registers for a second one: there the other waves cover.
-constexpr int kPipelinedChunks = 8;
-
+// One group per wave, the grid as large as that takes: the dispatcher's waves then cover each other's
+// loads, and workgroups that end early are replaced at once.  Looping over groups in 4096 workgroups
+// with the next group's loads in flight held 92 registers a lane and kept the waves in step: measured
+// on MI355X, from_dense's launch of fp16 [8, 32, 4096, 128] K and V (6 rotated tensors), with cached
+// stores 163 us, with non-temporal ones 150.5; 32768 workgroups without a loop
+// (44 registers) 129.6, 6.2 TB/s.
 template <int GF, int CH, typename XT, typename Map>
-__device__ __forceinline__ void quantize_groups_pipelined(const Map& map, int64_t ngroups, int rows, int D) {
+__device__ __forceinline__ void quantize_group_vec(const Map& map, int64_t groups, int rows, int D) {
   const int lane = threadIdx.x & (kWave - 1);
+  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  if (grp >= groups) return;
   const int n = rows * D;
   const LaneMap m = lane_map<GF>(n, D, lane);
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
-  int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  if (grp >= ngroups) return;
-  if constexpr (CH > kPipelinedChunks) {
-    for (; grp < ngroups; grp += waves) {
-      const GroupRef<XT> cur = map(grp);
-      RawGroup<CH, XT> raw;
-      load_raw(raw, cur.src, cur.valid_rows * D, n, m);
-      float x[CH][8];
-      unpack_group(raw, x);
-      quantize_any_regs<GF, CH>(x, cur.dst, cur.scale, cur.zero, n, m, lane);
-    }
-    return;
-  }
-  GroupRef<XT> cur = map(grp);
+  const GroupRef<XT> ref = map(grp);
   RawGroup<CH, XT> raw;
-  load_raw(raw, cur.src, cur.valid_rows * D, n, m);
-  for (;;) {
-    const int64_t nxt = grp + waves;
-    GroupRef<XT> ref_next{};
-    RawGroup<CH, XT> raw_next;
-    if (nxt < ngroups) {
-      ref_next = map(nxt);
-      load_raw(raw_next, ref_next.src, ref_next.valid_rows * D, n, m);
-    }
-    float x[CH][8];
-    unpack_group(raw, x);
-    quantize_any_regs<GF, CH>(x, cur.dst, cur.scale, cur.zero, n, m, lane);
-    if (nxt >= ngroups) break;
-    grp = nxt;
-    cur = ref_next;
-    raw = raw_next;
-  }
+  load_raw<GF>(raw, ref.src, ref.valid_rows * D, n, m);
+  float x[CH][8];
+  unpack_group(raw, x);
+  quantize_any_regs<GF, CH>(x, ref.dst, ref.scale, ref.zero, n, m, lane);
 }
 
 // Chunks of a group of `rows` rows when the vectorized quantizers apply (rounded up to an instantiated
@@ -586,7 +576,7 @@ __host__ __device__ constexpr int vec_chunks(int rows, int D) {
   return (D % 8 == 0 && (rows * D) % 512 == 0 && rows * D / 512 <= 8) ? rows * D / 512 : 0;
 }
 
-// x [outer, S, D] -> values [outer, nb, bs, D]; groups (o, block), vectorized and pipelined.
+// x [outer, S, D] -> values [outer, nb, bs, D]; groups (o, block), vectorized.
 template <int GF, int CH, typename XT>
 __global__ void __launch_bounds__(256)
 quantize_blocks_vec_kernel(const XT* x, int64_t outer, int S, int D, int bs, int nb, int8_t* values, float* scale,
@@ -598,28 +588,65 @@ quantize_blocks_vec_kernel(const XT* x, int64_t outer, int S, int D, int bs, int
     return GroupRef<XT>{x + ((size_t)o * S + (size_t)blk * bs) * D, min(S - blk * bs, bs), values + (size_t)grp * bs * D,
                         scale + (size_t)grp * per, zero ? zero + (size_t)grp * per : nullptr};
   };
-  quantize_groups_pipelined<GF, CH, XT>(map, outer * nb, bs, D);
+  quantize_group_vec<GF, CH, XT>(map, outer * nb, bs, D);
 }
 
-// dense [B, H, S, D] -> page store [P, H, page, D], vectorized and pipelined (see
-// quantize_pages_kernel).
+struct PageStore {
+  int8_t* values;
+  float* scale;
+  int16_t* zero;
+};
+
+// Dense K and V [B, H, S, D] -> page stores [P, H, page, D] (v null: K alone): physical page j holds
+// batch-major logical page page_src[j]; without a list it holds page j, or with `interleaved` page
+// (j % B) * nbps + j / B.  The launch also writes what the cache needs beside the pages, where asked
+// for: table[o] = the physical page of logical page o, and every request's length S.  One launch for
+// both tensors and both lists saves the gaps and the tails of five: measured on MI355X, from_dense
+// of fp16 [8, 32, 4096, 128] 160.7 -> 129.4 us (with one group per wave), of bf16 [4, 32, 2039, 128] to shuffled FP8 pages
+// 76.8 -> 55 us (torch.randperm's own launches remain).
+template <typename XT>
+struct PagesSource {
+  const XT* k;
+  const XT* v;
+  PageStore ks, vs;
+  const int64_t* page_src;
+  int64_t* table;
+  int64_t* lengths;
+  int64_t P;
+  int B, H, S, D, page, nbps, interleaved;
+};
+
+// Where group grp (K groups first, then V's; heads innermost) reads and writes.  I: index type; the
+// vectorized kernel takes 32 bits (the host keeps P * H < 2^31), a 64-bit division per group having
+// sat on the critical path to the next group's loads.
+template <int GF, typename I, typename XT>
+__device__ __forceinline__ GroupRef<XT> page_group(const PagesSource<XT>& s, int64_t group, int lane) {
+  const I per = (I)s.P * (I)s.H;
+  I g = sizeof(I) == 4 ? (I)__builtin_amdgcn_readfirstlane((int)group) : (I)group;  // one group per wave
+  const bool second = g >= per;
+  if (second) g -= per;
+  const I j = g / (I)s.H;
+  const int h = (int)(g - j * (I)s.H);
+  const I o = s.page_src ? (I)s.page_src[j] : (s.interleaved ? (j % (I)s.B) * (I)s.nbps + j / (I)s.B : j);
+  const I b = o / (I)s.nbps;
+  const int lb = (int)(o - b * (I)s.nbps);
+  if (h == 0 && !second && lane == 0) {
+    if (s.table) s.table[o] = (int64_t)j;
+    if (s.lengths && lb == 0) s.lengths[b] = s.S;
+  }
+  const PageStore st = second ? s.vs : s.ks;
+  const int params = group_params<GF>(s.page, s.D);
+  return GroupRef<XT>{(second ? s.v : s.k) + ((size_t)(b * (I)s.H + (I)h) * s.S + (size_t)lb * s.page) * s.D,
+                      min(s.S - lb * s.page, s.page), st.values + (size_t)g * s.page * s.D,
+                      st.scale + (size_t)g * params, st.zero ? st.zero + (size_t)g * params : nullptr};
+}
+
 template <int GF, int CH, typename XT>
 __global__ void __launch_bounds__(256)
-quantize_pages_vec_kernel(const XT* x, int H, int S, int D, int page, int nbps, const int64_t* page_src, int64_t P,
-                          int8_t* values, float* scale, int16_t* zero) {
-  // 32-bit index arithmetic (the host keeps P * H < 2^31): a 64-bit division per group sat on
-  // the critical path to the next group's loads
-  const int per = group_params<GF>(page, D);
-  auto map = [=](int64_t grp) {
-    const unsigned j = (unsigned)grp / (unsigned)H;
-    const int h = (int)((unsigned)grp - j * (unsigned)H);
-    const unsigned o = page_src ? (unsigned)page_src[j] : j;
-    const unsigned b = o / (unsigned)nbps;
-    const int lb = (int)(o - b * (unsigned)nbps);
-    return GroupRef<XT>{x + (((size_t)(b * H + h) * S) + (size_t)lb * page) * D, min(S - lb * page, page),
-                        values + (size_t)grp * page * D, scale + (size_t)grp * per, zero ? zero + (size_t)grp * per : nullptr};
-  };
-  quantize_groups_pipelined<GF, CH, XT>(map, P * H, page, D);
+quantize_pages_vec_kernel(const PagesSource<XT> s, int64_t groups) {
+  const int lane = threadIdx.x & (kWave - 1);
+  auto map = [&](int64_t grp) { return page_group<GF, unsigned>(s, grp, lane); };
+  quantize_group_vec<GF, CH, XT>(map, groups, s.page, s.D);
 }
 
 // x [outer, S, D] -> values [outer, nb, bs, D]; group = (o, block); rows past S read as 0.
@@ -642,26 +669,16 @@ quantize_blocks_kernel(const XT* x, int64_t outer, int S, int D, int bs, int nb,
   quantize_any_group<GF>(get, bs, D, values + (size_t)grp * bs * D, scale, zero, grp, lane);
 }
 
-// dense [B, H, S, D] -> page store [P, H, page, D]; physical page j holds batch-major
-// logical page src[j] (identity when src is null); rows past S read as 0.
-template <typename XT, int GF = kGfAffine>
+// quantize_pages_vec_kernel for any sizes and addresses; rows past S read as 0.
+template <typename XT, int GF>
 __global__ void __launch_bounds__(256)
-quantize_pages_kernel(const XT* x, int H, int S, int D, int page, int nbps, const int64_t* page_src, int64_t P,
-                      int8_t* values, float* scale, int16_t* zero) {
+quantize_pages_kernel(const PagesSource<XT> s, int64_t groups) {
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  if (grp >= P * H) return;
-  const int64_t j = grp / H;
-  const int h = (int)(grp - j * H);
-  const int64_t o = page_src ? page_src[j] : j;
-  const int64_t b = o / nbps;
-  const int lb = (int)(o - b * nbps);
-  const XT* src = x + ((size_t)(b * H + h) * S) * D;
-  auto get = [&](int r, int d) -> float {
-    const int s = lb * page + r;
-    return s < S ? to_f32(src[(size_t)s * D + d]) : 0.0f;
-  };
-  quantize_any_group<GF>(get, page, D, values + (size_t)grp * page * D, scale, zero, grp, lane);
+  if (grp >= groups) return;
+  const GroupRef<XT> ref = page_group<GF, int64_t>(s, grp, lane);
+  auto get = [&](int r, int d) -> float { return r < ref.valid_rows ? to_f32(ref.src[(size_t)r * s.D + d]) : 0.0f; };
+  quantize_any_group<GF>(get, s.page, s.D, ref.dst, ref.scale, ref.zero, 0, lane);
 }
 
 // Rewrite listed pages (see fs_update_pages_i8).
@@ -697,12 +714,6 @@ update_pages_kernel(const int8_t* in_values, const float* in_scale, const int16_
   const int64_t og = pg * H + h;
   quantize_group(get, page, D, out_values + (size_t)og * page * D, out_scale + og, out_zero + og, lane);
 }
-
-struct PageStore {
-  int8_t* values;
-  float* scale;
-  int16_t* zero;
-};
 
 // Prompt admission (see fs_write_prompt_i8): one request's K and V rows [H, src_tokens, D] into the
 // pages of a store, group = (K or V, logical page, head).  The page ids travel in the launch's
@@ -747,7 +758,7 @@ template <int CH, typename XT>
 __global__ void __launch_bounds__(256)
 prompt_pages_vec_kernel(const PromptSource<XT> s, int64_t groups, const PromptPages pages) {
   auto map = [&](int64_t grp) { return prompt_group(s, pages, grp); };
-  quantize_groups_pipelined<kGfAffine, CH, XT>(map, groups, s.page, s.D);
+  quantize_group_vec<kGfAffine, CH, XT>(map, groups, s.page, s.D);
 }
 
 template <typename XT>
@@ -971,16 +982,6 @@ dequantize_fp8_kernel(const uint8_t* values, const float* scale, int64_t outer, 
 
 static dim3 wave_grid(int64_t groups) { return dim3((unsigned)((groups + 3) / 4)); }
 
-// The pipelined vectorized quantizers loop over groups: at most 4096 workgroups of 4 waves (16 per
-// CU on 256 CUs), each wave taking every (waves)-th group.  Measured on MI355X, from_dense's page
-// quantizer on the metric workload's K tensor: 70.3 us with 4096, 71.5-71.9 with 2048 (0.905 and
-// 0.885 of the same box's 2:1 streaming copy).
-constexpr int64_t kVecQuantMaxBlocks = 4096;
-static dim3 vec_grid(int64_t groups) {
-  const int64_t blocks = (groups + 3) / 4;
-  return dim3((unsigned)(blocks < kVecQuantMaxBlocks ? blocks : kVecQuantMaxBlocks));
-}
-
 static bool is_pow2_chunks(int ch) { return ch == 1 || ch == 2 || ch == 4 || ch == 8; }
 
 // f(integral_constant<CH>) for the instantiated chunk counts of group_chunks.
@@ -1046,39 +1047,51 @@ static int launch_blocks(const char* what, const void* x, int x_dtype, int64_t o
       hipLaunchKernelGGL((quantize_blocks_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
     else
       by_chunks(ch, [&](auto c) {
-        hipLaunchKernelGGL((quantize_blocks_vec_kernel<GF, decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
+        hipLaunchKernelGGL((quantize_blocks_vec_kernel<GF, decltype(c)::value, XT>), wave_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
       });
   });
   return known ? check_launch(what) : set_error(FS_ERR_INVALID, std::string(what) + ": dtype code must be 0, 1 or 2");
 }
 
-// One launch of the page quantizer of format GF.
+// Where a page quantize launch places its pages, and the lists it writes beside them.
+struct PagePlan {
+  const int64_t* page_src;
+  int interleaved;
+  int64_t P;
+  int64_t* table;
+  int64_t* lengths;
+};
+
+// One launch of the page quantizer of format GF, for K and V (v null: K alone).
 template <int GF>
-static int launch_pages(const char* what, const void* x, int x_dtype, int batch, int H, int S, int D, int page,
-                        const int64_t* page_src, int64_t P, int8_t* values, float* scale, int16_t* zero,
-                        hipStream_t st) {
+static int launch_pages(const char* what, const void* k, const void* v, int x_dtype, int batch, int H, int S, int D,
+                        int page, const PagePlan& plan, PageStore ks, PageStore vs, hipStream_t st) {
   if (batch <= 0 || H <= 0 || S <= 0 || D <= 0 || page <= 0)
     return set_error(FS_ERR_INVALID, std::string(what) + ": sizes must be positive");
-  if (!x || !values || !scale || (!zero && GF != kGfFp8))
-    return set_error(FS_ERR_INVALID, std::string(what) + ": null pointer");
+  auto whole = [](const PageStore& p) { return p.values && p.scale && (p.zero || GF == kGfFp8); };
+  if (!k || !whole(ks) || (v && !whole(vs))) return set_error(FS_ERR_INVALID, std::string(what) + ": null pointer");
   const int nbps = (S + page - 1) / page;
-  if (P != (int64_t)batch * nbps)
+  if (plan.P != (int64_t)batch * nbps)
     return set_error(FS_ERR_INVALID, std::string(what) + ": num_pages must equal batch * ceil(seq_len / page)");
-  const int64_t groups = P * H;
-  const bool counted = groups <= 0x7fffffffLL;  // the vectorized kernel's index arithmetic is 32-bit
+  const bool counted = plan.P * H <= 0x7fffffffLL;  // the vectorized kernel's index arithmetic is 32-bit
   if (!counted && GF == kGfAffine)
     return set_error(FS_ERR_INVALID, std::string(what) + ": more than 2^31 (page, head) groups");
-  const bool aligned = counted && ((uintptr_t)x % 16) == 0 && ((uintptr_t)values % 8) == 0 &&
-                       (GF != kGfChannel || wide_params(scale, zero));
-  const int ch = aligned ? group_chunks(page, D, GF == kGfChannel || GF == kGfToken) : 0;
+  const int64_t groups = plan.P * H * (v ? 2 : 1);
+  auto aligned = [](const void* x, const PageStore& p) {
+    return ((uintptr_t)x % 16) == 0 && ((uintptr_t)p.values % 8) == 0 &&
+           (GF != kGfChannel || wide_params(p.scale, p.zero));
+  };
+  const int ch = counted && aligned(k, ks) && (!v || aligned(v, vs))
+                     ? group_chunks(page, D, GF == kGfChannel || GF == kGfToken) : 0;
   const bool known = by_dtype(x_dtype, [&](auto tag) {
     using XT = value_of<decltype(tag)>;
-    const XT* src = (const XT*)x;
+    const PagesSource<XT> s{(const XT*)k, (const XT*)v, ks, vs, plan.page_src, plan.table, plan.lengths, plan.P,
+                            batch, H, S, D, page, nbps, plan.interleaved};
     if (ch == 0)
-      hipLaunchKernelGGL((quantize_pages_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, src, H, S, D, page, nbps, page_src, P, values, scale, zero);
+      hipLaunchKernelGGL((quantize_pages_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, s, groups);
     else
       by_chunks(ch, [&](auto c) {
-        hipLaunchKernelGGL((quantize_pages_vec_kernel<GF, decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, src, H, S, D, page, nbps, page_src, P, values, scale, zero);
+        hipLaunchKernelGGL((quantize_pages_vec_kernel<GF, decltype(c)::value, XT>), wave_grid(groups), dim3(256), 0, st, s, groups);
       });
   });
   return known ? check_launch(what) : set_error(FS_ERR_INVALID, std::string(what) + ": dtype code must be 0, 1 or 2");
@@ -1119,8 +1132,9 @@ extern "C" int fs_dequantize_i8(const int8_t* values, const float* scale, const 
 extern "C" int fs_quantize_pages_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
                                     int page_size, const int64_t* page_src, int64_t num_pages, int8_t* values,
                                     float* scale, int16_t* zero, void* stream) {
-  return launch_pages<kGfAffine>("quantize_pages", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
-                                 num_pages, values, scale, zero, (hipStream_t)stream);
+  return launch_pages<kGfAffine>("quantize_pages", x, nullptr, x_dtype, batch, heads, seq_len, head_dim, page_size,
+                      PagePlan{page_src, 0, num_pages, nullptr, nullptr}, PageStore{values, scale, zero},
+                      PageStore{}, (hipStream_t)stream);
 }
 
 extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, int src_tokens, int length, int heads,
@@ -1157,7 +1171,7 @@ extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, i
         hipLaunchKernelGGL(prompt_pages_kernel<XT>, wave_grid(groups), dim3(256), 0, st, s, groups, ids);
       else
         by_chunks(ch, [&](auto c) {
-          hipLaunchKernelGGL((prompt_pages_vec_kernel<decltype(c)::value, XT>), vec_grid(groups), dim3(256), 0, st, s, groups, ids);
+          hipLaunchKernelGGL((prompt_pages_vec_kernel<decltype(c)::value, XT>), wave_grid(groups), dim3(256), 0, st, s, groups, ids);
         });
     });
     if (!known) return set_error(FS_ERR_INVALID, "write_prompt: dtype code must be 0, 1 or 2");
@@ -1287,8 +1301,9 @@ extern "C" int fs_quantize_fp8(const void* x, int x_dtype, int64_t outer, int se
 extern "C" int fs_quantize_pages_fp8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
                                      int page_size, const int64_t* page_src, int64_t num_pages, uint8_t* values,
                                      float* scale, int16_t* zero, void* stream) {
-  return launch_pages<kGfFp8>("quantize_pages_fp8", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
-                              num_pages, (int8_t*)values, scale, zero, (hipStream_t)stream);
+  return launch_pages<kGfFp8>("quantize_pages_fp8", x, nullptr, x_dtype, batch, heads, seq_len, head_dim, page_size,
+                      PagePlan{page_src, 0, num_pages, nullptr, nullptr}, PageStore{(int8_t*)values, scale, zero},
+                      PageStore{}, (hipStream_t)stream);
 }
 
 extern "C" int fs_dequantize_fp8(const uint8_t* values, const float* scale, int64_t outer, int n_blocks,
@@ -1321,13 +1336,32 @@ extern "C" int fs_quantize_i8_channel(const void* x, int x_dtype, int64_t outer,
 extern "C" int fs_quantize_pages_i8_channel(const void* x, int x_dtype, int batch, int heads, int seq_len,
                                             int head_dim, int page_size, const int64_t* page_src, int64_t num_pages,
                                             int8_t* values, float* scale, int16_t* zero, void* stream) {
-  return launch_pages<kGfChannel>("quantize_pages_channel", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
-                                  num_pages, values, scale, zero, (hipStream_t)stream);
+  return launch_pages<kGfChannel>("quantize_pages_channel", x, nullptr, x_dtype, batch, heads, seq_len, head_dim, page_size,
+                      PagePlan{page_src, 0, num_pages, nullptr, nullptr}, PageStore{values, scale, zero},
+                      PageStore{}, (hipStream_t)stream);
 }
 
 extern "C" int fs_quantize_pages_sym_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
                                         int page_size, const int64_t* page_src, int64_t num_pages, int8_t* values,
                                         float* scale, int16_t* zero, void* stream) {
-  return launch_pages<kGfToken>("quantize_pages_symmetric", x, x_dtype, batch, heads, seq_len, head_dim, page_size, page_src,
-                                num_pages, values, scale, zero, (hipStream_t)stream);
+  return launch_pages<kGfToken>("quantize_pages_symmetric", x, nullptr, x_dtype, batch, heads, seq_len, head_dim, page_size,
+                      PagePlan{page_src, 0, num_pages, nullptr, nullptr}, PageStore{values, scale, zero},
+                      PageStore{}, (hipStream_t)stream);
+}
+
+extern "C" int fs_build_cache(const void* k, const void* v, int src_dtype, int kv_format, int batch, int heads,
+                              int seq_len, int head_dim, int page_size, const int64_t* page_src, int interleaved,
+                              int64_t num_pages, void* k_values, float* k_scale, int16_t* k_zero, void* v_values,
+                              float* v_scale, int16_t* v_zero, int64_t* block_table, int64_t* lengths, void* stream) {
+  if (!v) return set_error(FS_ERR_INVALID, "build_cache: null pointer");
+  const PagePlan plan{page_src, interleaved, num_pages, block_table, lengths};
+  const PageStore ks{(int8_t*)k_values, k_scale, k_zero}, vs{(int8_t*)v_values, v_scale, v_zero};
+  const hipStream_t st = (hipStream_t)stream;
+  switch (kv_format) {
+    case 0: return launch_pages<kGfAffine>("build_cache", k, v, src_dtype, batch, heads, seq_len, head_dim, page_size, plan, ks, vs, st);
+    case 1: return launch_pages<kGfFp8>("build_cache", k, v, src_dtype, batch, heads, seq_len, head_dim, page_size, plan, ks, vs, st);
+    case 2: return launch_pages<kGfChannel>("build_cache", k, v, src_dtype, batch, heads, seq_len, head_dim, page_size, plan, ks, vs, st);
+    case 3: return launch_pages<kGfToken>("build_cache", k, v, src_dtype, batch, heads, seq_len, head_dim, page_size, plan, ks, vs, st);
+    default: return set_error(FS_ERR_INVALID, "build_cache: kv_format must be 0 to 3");
+  }
 }

@@ -6,7 +6,7 @@ quant block == page, i.e. ``values [P, H, 1, page, D]`` and ``scale/zero
 maps logical pages to physical ones.
 
 On GPU every quantized write goes through the HIP page kernels:
-``fs_quantize_pages_i8`` for ``from_dense`` and ``fs_update_pages_i8`` for
+``fs_build_cache`` for ``from_dense`` and ``fs_update_pages_i8`` for
 ``append`` (whole-store requantization, as the reference does) and for the
 allocator's append writes (only the touched pages), ``fs_write_prompt_i8`` for its prompts.  Host bookkeeping —
 free list, tables, lengths — stays in Python like the reference's.
@@ -27,6 +27,9 @@ from .quant import (FP8_DTYPE, QuantizedTensor, dequantize_int8_per_block, estim
                     quantize_int8_symmetric_per_token)
 
 _SCALE_FLOOR = 1.0e-8  # quantizing an all-zero block gives int8 -128, scale fp32(1e-8), zero 0
+
+
+_FORMAT_CODES = {"affine_block": 0, "fp8_block": 1, "affine_channel": 2, "symmetric_token": 3}  # fs_build_cache
 
 
 def _normalize_device(device: torch.device | str) -> torch.device:
@@ -464,27 +467,34 @@ class PagedKVCache:
         batch, heads, seq_len, head_dim = (int(s) for s in k.shape)
         blocks_per_seq = (seq_len + block_size - 1) // block_size
         total = batch * blocks_per_seq
-        perm = _layout_permutation(pattern, batch, blocks_per_seq, layout_seed, k.device)
-        if perm is None:
-            block_table = torch.arange(total, dtype=torch.int64, device=k.device).reshape(batch, blocks_per_seq)
-        else:
-            inverse = torch.empty_like(perm)
-            inverse[perm] = torch.arange(total, dtype=torch.int64, device=k.device)
-            block_table = inverse.reshape(batch, blocks_per_seq)
+        on_gpu = k.device.type == "cuda"
+        perm = None  # on the GPU the quantizing launch places interleaved pages and writes the table itself
+        if not on_gpu or pattern in {"shuffled", "random"}:
+            perm = _layout_permutation(pattern, batch, blocks_per_seq, layout_seed, k.device)
 
-        if lengths is None:
-            effective_lengths = torch.full((batch,), seq_len, dtype=torch.int64, device=k.device)
-        else:
+        effective_lengths = None
+        if lengths is not None:
             effective_lengths = lengths.to(device=k.device, dtype=torch.int64).contiguous()
             if effective_lengths.ndim != 1 or effective_lengths.shape[0] != batch:
                 raise ValueError("lengths must be [batch]")
             if bool((effective_lengths < 0).any().item()) or bool((effective_lengths > seq_len).any().item()):
                 raise ValueError("lengths must lie in [0, seq_len]")
 
-        if k.device.type == "cuda":
-            k_quant = cls._quantize_pages(k, block_size, perm, total, kv_format)
-            v_quant = cls._quantize_pages(v, block_size, perm, total, kv_format)
+        if on_gpu:
+            k_quant, v_quant, block_table, full_lengths = cls._build_hip(k, v, block_size, perm,
+                                                                         pattern == "interleaved", kv_format,
+                                                                         lengths is None)
+            if effective_lengths is None:
+                effective_lengths = full_lengths
         else:
+            if perm is None:
+                block_table = torch.arange(total, dtype=torch.int64).reshape(batch, blocks_per_seq)
+            else:
+                inverse = torch.empty_like(perm)
+                inverse[perm] = torch.arange(total, dtype=torch.int64)
+                block_table = inverse.reshape(batch, blocks_per_seq)
+            if effective_lengths is None:
+                effective_lengths = torch.full((batch,), seq_len, dtype=torch.int64)
             k_pages, v_pages = cls._physical_pages(k, block_size, perm), cls._physical_pages(v, block_size, perm)
             if kv_format == "symmetric_token":
                 k_quant, v_quant = map(quantize_int8_symmetric_per_token, (k_pages, v_pages))
@@ -506,22 +516,28 @@ class PagedKVCache:
         return pages if perm is None else pages[perm].contiguous()
 
     @staticmethod
-    def _quantize_pages(x: torch.Tensor, block_size: int, perm: torch.Tensor | None, total: int,
-                        kv_format: str) -> QuantizedTensor:
+    def _build_hip(k: torch.Tensor, v: torch.Tensor, block_size: int, perm: torch.Tensor | None, interleaved: bool,
+                   kv_format: str, full: bool):
+        """Both stores, the block table and (``full``) the lengths of a cache, by one ``fs_build_cache`` launch."""
+
+        if v.device != k.device:
+            raise ValueError("k and v must be on the same device")
         lib = _lib.require()
-        batch, heads, seq_len, head_dim = (int(s) for s in x.shape)
-        src = _src_for_kernel(x.detach())
-        values, scale, zero = _empty_page_store(total, heads, block_size, head_dim, x.device, kv_format)
-        page_src = None if perm is None else perm.to(torch.int64).contiguous()
-        quantize_pages = {"affine_block": lib.fs_quantize_pages_i8, "fp8_block": lib.fs_quantize_pages_fp8,
-                          "affine_channel": lib.fs_quantize_pages_i8_channel,
-                          "symmetric_token": lib.fs_quantize_pages_sym_i8}[kv_format]
-        _lib.check(quantize_pages(
-            src.data_ptr(), _lib.dtype_code(src.dtype), batch, heads, seq_len, head_dim, block_size,
-            _lib.ptr(page_src), total, values.data_ptr(), scale.data_ptr(), zero.data_ptr(),
-            _lib.stream_ptr(x.device)))
-        return QuantizedTensor(values, scale, zero, 1 if kv_format == "symmetric_token" else block_size,
-                               (total, heads, block_size, head_dim))
+        batch, heads, seq_len, head_dim = (int(s) for s in k.shape)
+        ks, vs = _src_for_kernel(k.detach()), _src_for_kernel(v.detach())
+        if ks.dtype != vs.dtype:  # exact: the quantizers compute in float32
+            ks, vs = ks.to(torch.float32), vs.to(torch.float32)
+        blocks_per_seq = (seq_len + block_size - 1) // block_size
+        total, dev = batch * blocks_per_seq, k.device
+        stores = [_empty_page_store(total, heads, block_size, head_dim, dev, kv_format) for _ in range(2)]
+        table = torch.empty((batch, blocks_per_seq), dtype=torch.int64, device=dev)
+        lengths = torch.empty((batch,), dtype=torch.int64, device=dev) if full else None
+        _lib.check(lib.fs_build_cache(
+            ks.data_ptr(), vs.data_ptr(), _lib.dtype_code(ks.dtype), _FORMAT_CODES[kv_format], batch, heads, seq_len,
+            head_dim, block_size, _lib.ptr(perm), int(interleaved), total, *(t.data_ptr() for s in stores for t in s),
+            table.data_ptr(), _lib.ptr(lengths), _lib.stream_ptr(dev)))
+        quant_block, shape = (1 if kv_format == "symmetric_token" else block_size), (total, heads, block_size, head_dim)
+        return (*(QuantizedTensor(*s, quant_block, shape) for s in stores), table, lengths)
 
     def to_dense(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """Dequantize the store and gather ``[batch, heads, max_seq_len, dim]`` (paged.py:421-461)."""

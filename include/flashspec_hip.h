@@ -336,6 +336,18 @@ int fs_quantize_pages_sym_i8(const void* x, int x_dtype, int batch, int heads, i
                              int page_size, const int64_t* page_src, int64_t num_pages,
                              int8_t* values, float* scale, int16_t* zero, void* stream);
 
+/* A whole paged cache from dense k and v [batch, heads, seq_len, head_dim] in one launch (replaces
+ * reference paged.py:302-419): both stores as the fs_quantize_pages_* entry of kv_format (0 affine
+ * INT8, 1 FP8 E4M3, 2 per-channel INT8, 3 symmetric per-token INT8) writes them, and, where not
+ * NULL, block_table [batch, ceil(seq_len / page_size)] and lengths [batch] (all seq_len).  Pages are
+ * placed by page_src (physical page j holds batch-major logical page page_src[j], a permutation), or
+ * without it in batch-major order, or with `interleaved` in logical-page-major order. */
+int fs_build_cache(const void* k, const void* v, int src_dtype, int kv_format, int batch, int heads,
+                   int seq_len, int head_dim, int page_size, const int64_t* page_src, int interleaved,
+                   int64_t num_pages, void* k_values, float* k_scale, int16_t* k_zero,
+                   void* v_values, float* v_scale, int16_t* v_zero,
+                   int64_t* block_table, int64_t* lengths, void* stream);
+
 /*
  * FP8 E4M3 (OCP "e4m3fn") KV format: per block of block_size tokens x head_dim (zero-padded
  * like fs_quantize_i8), one fp32 scale and no zero point:

@@ -175,6 +175,32 @@ def test_build_matches_the_portable_path_bit_exact(kv_format, dim, page, seq, dt
         assert_same_store(cache.v_quant, ref.v_quant, "v")
 
 
+@pytest.mark.parametrize("pattern", ["contiguous", "interleaved", "shuffled"])
+@pytest.mark.parametrize("batch,seq,dim", [(1, 16, 128), (5, 33, 128), (3, 50, 36)])
+def test_build_writes_table_and_lengths(pattern, batch, seq, dim):
+    """Both page kernels place the pages, write the table and, without given lengths, the lengths."""
+
+    announce(f"from_dense table and lengths {pattern} B{batch} S{seq} D{dim}")
+    k, v = randn((batch, 2, seq, dim), 1), randn((batch, 2, seq, dim), 2, torch.float32)  # two dtypes
+    got = fa.PagedKVCache.from_dense(k.to(DEV), v.to(DEV), 16, block_table_pattern=pattern, layout_seed=3)
+    given = fa.PagedKVCache.from_dense(k.to(DEV), v.to(DEV), 16, block_table_pattern=pattern, layout_seed=3,
+                                       lengths=torch.arange(1, batch + 1, device=DEV))
+    torch.cuda.synchronize()
+    n = batch * -(-seq // 16)
+    if pattern == "shuffled":
+        g = torch.Generator(device=DEV)
+        g.manual_seed(3)
+        want = torch.argsort(torch.randperm(n, generator=g, device=DEV)).cpu().reshape(batch, -1)
+    else:
+        want = fa.PagedKVCache.from_dense(k, v, 16, block_table_pattern=pattern).block_table
+    assert torch.equal(got.block_table.cpu(), want) and torch.equal(given.block_table.cpu(), want)
+    assert got.lengths.tolist() == [seq] * batch and given.lengths.tolist() == list(range(1, batch + 1))
+    for quant, x in ((got.k_quant, k), (got.v_quant, v)):
+        ref = fa.quantize_int8_per_block(x, 16)
+        assert torch.equal(quant.values.cpu()[want][:, :, :, 0], ref.values.permute(0, 2, 1, 3, 4))
+        assert torch.equal(quant.scale.cpu()[want].reshape(batch, -1, 2), ref.scale[..., 0, 0].permute(0, 2, 1))
+
+
 @pytest.mark.parametrize("kv_format", FORMATS)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("dim", [80, 128])
