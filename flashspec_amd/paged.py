@@ -542,6 +542,8 @@ class PagedKVCache:
     def to_dense(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """Dequantize the store and gather ``[batch, heads, max_seq_len, dim]`` (paged.py:421-461)."""
 
+        if self.k_quant.device.type == "cuda" and self._readable():
+            return self._to_dense_hip()
         physical_k = dequantize_int8_per_block(self.k_quant, dtype=torch.float32)
         physical_v = dequantize_int8_per_block(self.v_quant, dtype=torch.float32)
         table = self.block_table.clamp_min(0)
@@ -551,6 +553,50 @@ class PagedKVCache:
                     .reshape(self.batch_size, self.num_heads, -1, self.head_dim)[..., : self.max_seq_len, :])
 
         return gather(physical_k), gather(physical_v)
+
+    def _readable(self) -> bool:
+        """Whether both stores are plain paged stores ([pages, heads, blocks, block, head_dim], parameters of the
+        usual types) under an integer table, all on one GPU, with something to read: what ``fs_read_cache`` takes."""
+
+        kq, table = self.k_quant, self.block_table
+        if table.ndim != 2 or table.dtype not in (torch.int32, torch.int64) or table.device != kq.device:
+            return False
+        if min(table.numel(), int(self.max_seq_len), kq.values.numel()) <= 0:
+            return False
+        for q in (kq, self.v_quant):
+            if q.values.ndim != 5 or len(q.original_shape) != 4 or q.device != kq.device or \
+                    q.values.dtype not in (torch.int8, FP8_DTYPE) or q.scale.dtype != torch.float32 or \
+                    q.zero_point.dtype != torch.int16:
+                return False
+            pages, heads, blocks, rows, dim = q.values.shape
+            shape = tuple(int(n) for n in q.original_shape)
+            params = pages * heads * blocks * (dim if is_per_channel(q) else 1)
+            if shape != tuple(kq.original_shape) or (pages, heads, dim) != (shape[0], shape[1], shape[3]) or \
+                    not 0 < shape[2] <= blocks * rows or (is_per_channel(q) and is_fp8(q)) or \
+                    q.scale.numel() != params or q.zero_point.numel() != params:
+                return False
+        return True
+
+    def _to_dense_hip(self) -> Tuple[torch.Tensor, torch.Tensor]:
+        """Both stores dequantized straight to ``[batch, heads, max_seq_len, dim]`` (one launch for stores alike)."""
+
+        lib = _lib.require()
+        kq, vq, table = self.k_quant, self.v_quant, self.block_table.contiguous()
+        pages, heads, page, dim = (int(n) for n in kq.original_shape)
+        batch, cols = (int(n) for n in table.shape)
+        seq = min(int(self.max_seq_len), cols * page)
+        outs = [torch.empty((batch, heads, seq, dim), dtype=torch.float32, device=kq.device) for _ in range(2)]
+        k_code, v_code = (1 if is_fp8(q) else (2 if is_per_channel(q) else 0) for q in (kq, vq))
+        alike = kq.values.shape == vq.values.shape and k_code == v_code
+        kt, vt = ([t.contiguous() for t in (q.values, q.scale, q.zero_point)] for q in (kq, vq))
+        for code, first, second, out, out2 in ([(k_code, kt, vt, *outs)] if alike else
+                                               [(k_code, kt, None, outs[0], None), (v_code, vt, None, outs[1], None)]):
+            ptrs = [t.data_ptr() for t in first] + ([None] * 3 if second is None else [t.data_ptr() for t in second])
+            blocks, rows = (int(n) for n in first[0].shape[2:4])
+            _lib.check(lib.fs_read_cache(
+                *ptrs, code, table.data_ptr(), table.element_size(), cols, batch, heads, seq, dim, pages, page, blocks,
+                rows, out.data_ptr(), _lib.ptr(out2), 0, _lib.stream_ptr(kq.device)))
+        return outs[0], outs[1]
 
     def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> "PagedKVCache":
         """Append ``[batch, heads, tokens, dim]`` to every row; returns a new cache (paged.py:463-557).

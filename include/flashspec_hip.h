@@ -348,6 +348,18 @@ int fs_build_cache(const void* k, const void* v, int src_dtype, int kv_format, i
                    void* v_values, float* v_scale, int16_t* v_zero,
                    int64_t* block_table, int64_t* lengths, void* stream);
 
+/* A paged cache read back as dense rows (replaces reference paged.py:421-461): k_out and v_out
+ * [batch, heads, seq_len, head_dim], row s of request b and head h being row s % page_size of page
+ * block_table[b, s / page_size], dequantized.  A negative table entry reads page 0 (the reference clamps
+ * it); an entry past num_pages reads as NaN.  kv_format: 0 INT8 with one parameter per quant block, 1 FP8
+ * E4M3 (zero points unused), 2 per-channel INT8.  Values are [num_pages, heads, n_blocks, quant_block,
+ * head_dim] with n_blocks * quant_block >= page_size.  v_values may be NULL (K alone). */
+int fs_read_cache(const void* k_values, const float* k_scale, const int16_t* k_zero,
+                  const void* v_values, const float* v_scale, const int16_t* v_zero, int kv_format,
+                  const void* block_table, int table_index_bytes, int table_cols,
+                  int batch, int heads, int seq_len, int head_dim, int64_t num_pages, int page_size,
+                  int n_blocks, int quant_block, void* k_out, void* v_out, int out_dtype, void* stream);
+
 /*
  * FP8 E4M3 (OCP "e4m3fn") KV format: per block of block_size tokens x head_dim (zero-padded
  * like fs_quantize_i8), one fp32 scale and no zero point:

@@ -237,6 +237,70 @@ def test_infinities_nan_and_scratch_ranges_match_the_general_path(dtype):
     assert torch.equal(a.zero_point, b.zero_point)
 
 
+# 4 values a lane (D 128, 36, 256, 24) and one (34, 7); pages of one wave, of several (D 256, 64 rows)
+# and of a part; whole and cut last pages; more table columns than tokens; -1 entries
+@pytest.mark.parametrize("kv_format", FORMATS)
+@pytest.mark.parametrize("heads,dim,page,seq,table_dtype", [
+    (2, 128, 16, 300, torch.int64),
+    (3, 36, 16, 33, torch.int32),
+    (2, 256, 64, 130, torch.int64),
+    (2, 24, 8, 64, torch.int32),
+    (2, 34, 16, 40, torch.int64),
+    (1, 7, 4, 10, torch.int64),
+])
+def test_to_dense_matches_the_portable_path(kv_format, heads, dim, page, seq, table_dtype):
+    announce(f"to_dense {kv_format} H{heads} D{dim} page{page} S{seq} {table_dtype}")
+    k, v = randn((3, heads, seq, dim), 1) * 2.0, randn((3, heads, seq, dim), 2)
+    ref = fa.PagedKVCache.from_dense(k, v, page, block_table_pattern="interleaved", kv_format=kv_format)
+    table = ref.block_table.clone()
+    table[1, -1] = -1
+    table = torch.cat([table, torch.full((3, 1), -1)], dim=1)
+    for span in (seq, seq - 3, (table.shape[1] - 1) * page + 1, 10 * table.shape[1] * page):
+        want = fa.PagedKVCache(ref.k_quant, ref.v_quant, table, ref.lengths, page, span).to_dense()
+
+        def moved(q):
+            return fa.QuantizedTensor(q.values.to(DEV), q.scale.to(DEV), q.zero_point.to(DEV), q.block_size,
+                                      q.original_shape)
+
+        got = fa.PagedKVCache(moved(ref.k_quant), moved(ref.v_quant), table.to(DEV, table_dtype),
+                              ref.lengths.to(DEV), page, span).to_dense()
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert a.dtype == torch.float32 and a.shape == b.shape
+            assert torch.equal(a.cpu().view(torch.int32), b.contiguous().view(torch.int32))
+
+
+def test_to_dense_of_stores_that_differ_and_of_quant_blocks_in_a_page():
+    announce("to_dense: INT8 K with 8-token blocks, FP8 V, page 20 over 16-token blocks")
+    x = randn((6, 2, 32, 64), 3)
+    table = torch.tensor([[5, 0, 3], [1, 2, 4]])
+    k, v = fa.quantize_int8_per_block(x, 8), fa.quantize_fp8_per_block(x, 32)
+    y = randn((6, 2, 20, 64), 4)
+    short = fa.quantize_int8_per_block(y, 16)  # two blocks of 16 hold a page of 20
+    for kq, vq, page in ((k, v, 32), (short, short, 20)):
+        want = fa.PagedKVCache(kq, vq, table, torch.tensor([70, 60]), page, 3 * page - 7).to_dense()
+        on = [fa.QuantizedTensor(q.values.to(DEV), q.scale.to(DEV), q.zero_point.to(DEV), q.block_size,
+                                 q.original_shape) for q in (kq, vq)]
+        got = fa.PagedKVCache(on[0], on[1], table.to(DEV), torch.tensor([70, 60], device=DEV), page,
+                              3 * page - 7).to_dense()
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a.cpu(), b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,block,seq", [(128, 16, 301), (34, 8, 21), (3000, 4, 9)])
+def test_dequantize_matches_the_portable_path(dtype, dim, block, seq):
+    announce(f"dequantize D{dim} block{block} S{seq} {dtype}")
+    x = randn((2, 3, seq, dim), 5)
+    for quantize in (fa.quantize_int8_per_block, fa.quantize_fp8_per_block):
+        q = quantize(x, block)
+        on = fa.QuantizedTensor(q.values.to(DEV), q.scale.to(DEV), q.zero_point.to(DEV), block, q.original_shape)
+        got, want = fa.dequantize_int8_per_block(on, dtype), fa.dequantize_int8_per_block(q, dtype)
+        torch.cuda.synchronize()
+        assert torch.equal(got.cpu(), want)
+
+
 def test_prompt_entry_rejects_bad_sizes():
     lib = _lib.require()
     ids = (np.zeros(4, dtype=np.int32)).ctypes.data
