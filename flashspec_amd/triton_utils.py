@@ -321,6 +321,68 @@ def plan_splits(seq_len: int, rows: int, block_n: int, cu_count: int, *, tiled: 
     return split_tiles, math.ceil(tiles / split_tiles), waves
 
 
+# The default plan of the tiled path (no knob set; plan_splits serves the knobs).  Measured on MI355X
+# over 5 KV formats and head_dims, 8 to 384 rows of 16 to 1024 tiles, every split count and 4 / 8 / 16
+# waves (kernel time, us):
+# * Splits never put more workgroups than CUs: a second, nearly empty round costs a whole split.
+#   B5 H32 S4096 D128 (160 rows): 2 splits 41.0, unsplit 29.8; B3 (96 rows): 3 splits 30.3, 2 splits 20.6.
+# * Rows on over half of the CUs but not all take splits of 4 waves from PLAN_SLOT_TILES on, two
+#   workgroups a CU: rows of unlike length then spread (160 rows of up to 313 tiles, per-channel: whole
+#   62.9, 2 splits of 8 waves 48.2; 160 full rows of 256 tiles: 56.0, 61.2 and, 3 of 4 waves, 43.8).
+# * A row takes at most sqrt(tiles) / 2 splits: the last split's merge grows with their number.  8 rows
+#   of 1024 tiles: 32 splits 20.6, 16 splits 16.3; 8 rows of 128 tiles: 16 splits 11.4, 4 splits 8.5.
+# * Rows under PLAN_MIN_TILES stay whole (64 rows of 32 tiles: 4 splits 7.8, unsplit 6.6); 256-dim and
+#   per-channel tiles, whose tiles cost about twice as much, from half of that.
+# * 8 waves per workgroup, two tiles a wave at least (four at 256 dims or with more rows than CUs),
+#   merged in the launch: splits on 16 waves paid a workspace and a merge launch (B2 S8192 per-token
+#   27.4, on 8 waves 25.2).
+# * Light tiles (LIGHT_WAVES) take 4 waves where a workgroup lands on nearly every CU and a wave keeps
+#   16 to 64 tiles (256 rows of 256 tiles: 42.1, on 8 waves 44.2; 224 rows: 39.9 and 38.6).
+# * As many rows as CUs or more: 8 waves, and 16 from PLAN_LONG_TILES on, where rows of unlike length
+#   leave the last round to few workgroups (512 rows of 64 tiles: 24.1, on 16 waves 26.6; of up to 188 tiles,
+#   falling to 1/16: 41.5 and 38.2).
+PLAN_MIN_TILES = 64
+PLAN_LONG_TILES = 128
+PLAN_SLOT_TILES = 256
+PLAN_WAVES = 8
+PLAN_LIGHT_MIN_FILL = 0.9
+
+
+def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_waves: int = MAX_TILED_WAVES,
+              tile_group: int = 1, light: bool = False, per_channel: bool = False) -> tuple[int, int, int]:
+    """``(split_tiles, max_splits, waves_per_block)`` of a tiled decode launch (rule above); arguments as
+    for ``plan_splits``."""
+
+    tiles = max(1, math.ceil(seq_len / TILE_TOKENS))
+    grp = max(1, tile_group)
+    groups = math.ceil(tiles / grp)
+    costly = head_dim > 128 or per_channel
+    n = 1
+    if tiles >= (PLAN_MIN_TILES // 2 if costly else PLAN_MIN_TILES):
+        n = max(1, min(cu_count // max(1, rows), int(math.sqrt(tiles) / 2), groups))
+    paired = n == 1 and cu_count < 2 * rows < 2 * cu_count and tiles >= PLAN_SLOT_TILES
+    if paired:
+        n = min(2 * cu_count // rows, groups)
+    split_groups = math.ceil(groups / n)
+    n = math.ceil(groups / split_groups)
+    split = split_groups * grp
+    per_wave = max(4 if head_dim > 128 or rows > cu_count else 2, grp)
+    waves = 1
+    while waves < min(PLAN_WAVES, max_waves) and 2 * waves * per_wave <= split:
+        waves *= 2
+    if paired or (light and grp == 1 and PLAN_LIGHT_MIN_FILL * cu_count < rows * n <= cu_count and
+                 LIGHT_MIN_SPLIT_TILES <= split <= LIGHT_WAVES * MAX_TILES_PER_WAVE):
+        waves = min(waves, LIGHT_WAVES)
+    elif rows >= cu_count and split >= PLAN_LONG_TILES:
+        waves = max_waves
+    while waves < max_waves and split_groups > MAX_TILES_PER_WAVE // grp * waves:
+        waves *= 2
+    cap = MAX_TILES_PER_WAVE // grp * waves
+    if split_groups > cap:
+        split_groups = math.ceil(groups / math.ceil(groups / cap))
+    return split_groups * grp, math.ceil(tiles / (split_groups * grp)), waves
+
+
 # One 8-wave workgroup of the multi-query kernel holds a CU (its ~140 registers per lane leave
 # room for 3 waves per SIMD): the plan splits only while the grid fits one workgroup per CU.
 # Measured on MI355X, B4 H32 S4096 D128, 16 nodes: 2 splits (256 workgroups) 33.5 us,
@@ -402,7 +464,8 @@ def torch_device(device):
 @functools.lru_cache(maxsize=512)
 def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, quant_block: int, dev_type: str,
                         dev_index, per_channel: bool, light: bool, contiguous: bool, knobs: tuple):
-    """`knobs` only keys the cache: the helpers below read the same values from the environment."""
+    """`knobs` keys the cache and says whether any is set; the helpers below read the same values from the
+    environment."""
 
     import torch
 
@@ -426,6 +489,11 @@ def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, 
     # the default plan's ceiling (a forced wave count keeps only the register limit above)
     if contiguous and tiled and not per_channel and head_dim == 64:
         max_waves = min(max_waves, CONTIGUOUS_D64_WAVES)
-    split_tiles, max_splits, waves = plan_splits(seq_len, rows, block_n, device_cu_count(device), tiled=tiled,
-                                                 waves=waves, max_waves=max_waves, tile_group=group, light=light)
+    if tiled and not any(knobs):
+        split_tiles, max_splits, waves = plan_rows(seq_len, rows, head_dim, device_cu_count(device),
+                                                   max_waves=max_waves, tile_group=group, light=light,
+                                                   per_channel=per_channel)
+    else:
+        split_tiles, max_splits, waves = plan_splits(seq_len, rows, block_n, device_cu_count(device), tiled=tiled,
+                                                     waves=waves, max_waves=max_waves, tile_group=group, light=light)
     return tiled, waves, split_tiles, max_splits, block_n
