@@ -37,7 +37,8 @@ from . import _lib
 from .paged import PagedKVAllocator, PagedKVCache
 from .quant import QuantizedTensor, dequantize_int8_per_block, quantize_int8_per_block
 from .runtime import device_name, resolve_device, resolve_dtype, synchronize
-from .triton_paged import paged_quant_attention_triton
+from .triton_paged import _run_paged_quant_attention_triton, paged_quant_attention_triton
+from .triton_utils import MERGE_MAX_WAVES, device_cu_count, launch_plan, merge_area
 
 DTYPE_CHOICES = ["auto", "float16", "fp16", "bfloat16", "bf16", "float32", "fp32"]
 
@@ -415,8 +416,6 @@ class DecodeBatch:
         with the requests dispatched longest first; the output does not depend on the order)."""
 
         if q.device.type == "cuda" and q.device == self.device:
-            from .triton_paged import _run_paged_quant_attention_triton
-
             return _run_paged_quant_attention_triton(q, self.cache(), return_stats=return_stats,
                                                      request_order=self._order)
         return paged_quant_attention_triton(q, self.cache(), return_stats=return_stats)
@@ -444,13 +443,11 @@ class DecodeBatch:
         a = self.allocator
         return (self._open and self.device.type == "cuda" and self.page == 16 and a.k_quant.block_size == 16
                 and a.head_dim in (64, 128, 256) and q.dtype == k_new.dtype == v_new.dtype
-                and tuple(q.shape) == (len(self._requests), a.heads, a.head_dim) and q.device == self.device
+                and q.shape == (len(self._requests), a.heads, a.head_dim) and q.device == self.device
                 and self.steps_done < self.max_new_tokens)
 
     def _fused_plan(self, q):
         """(max_seq_len, launch plan) of a one-launch step whose grid fits one workgroup per CU, else None."""
-
-        from .triton_utils import device_cu_count, launch_plan
 
         a = self.allocator
         # every row covers its appended token: the longest request after the step, in whole pages
@@ -463,8 +460,6 @@ class DecodeBatch:
         return max_seq_len, plan
 
     def _step_fused(self, q, k_new, v_new, fused_plan) -> torch.Tensor:
-        from .triton_utils import MERGE_MAX_WAVES, merge_area
-
         n, a = len(self._requests), self.allocator
         for t in (k_new, v_new):
             if t.shape != (n, a.heads, 1, a.head_dim):

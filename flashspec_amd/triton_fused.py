@@ -24,7 +24,7 @@ from .triton_utils import (
     MERGE_MAX_WAVES,
     kv_format_code,
     launch_plan,
-    layout_checked,
+    layout_facts,
     merge_area,
     remember_layout,
     resolve_block_n as _resolve_block_n,
@@ -113,24 +113,23 @@ def _run_fused_dequant_attention_triton(q: torch.Tensor, k_quant: QuantizedTenso
                 k_quant.zero_point.numel(), vv_.data_ptr(), vv_.numel(), v_quant.scale.numel(),
                 v_quant.zero_point.numel(), None if lengths is None else (lengths.shape, lengths.device, lengths.dtype))
     memo = k_quant.__dict__.get("_fs_v_ref")
-    if not (layout_checked(k_quant, memo_key) and memo is not None and memo() is v_quant):
+    facts = layout_facts(k_quant, memo_key) if memo is not None and memo() is v_quant else None
+    if facts is None:
         _validate_triton_fused_inputs(q, k_quant, v_quant, lengths)
-        remember_layout(k_quant, memo_key)
+        batch, heads, head_dim = (int(s) for s in q.shape)
+        facts = (batch, heads, head_dim, int(k_quant.original_shape[-2]), int(kv_.shape[-3]), int(k_quant.block_size),
+                 q.dtype in (torch.float16, torch.bfloat16), _lib.dtype_code(q.dtype),
+                 1.0 / math.sqrt(float(head_dim)))
+        remember_layout(k_quant, memo_key, facts)
         object.__setattr__(k_quant, "_fs_v_ref", weakref.ref(v_quant))
+    batch, heads, head_dim, seq_len, n_blocks, block_size, light, qcode, sm_scale = facts
+    fp8, per_channel = kv_.dtype == FP8_DTYPE, k_quant.scale.shape[-1] == head_dim > 1
     lib = _lib.require()
     q_c = q.contiguous()
-    kv = [t.contiguous() for t in (k_quant.values, k_quant.scale, k_quant.zero_point,
-                                    v_quant.values, v_quant.scale, v_quant.zero_point)]
+    kv = [t.contiguous() for t in (kv_, k_quant.scale, k_quant.zero_point, vv_, v_quant.scale, v_quant.zero_point)]
     lengths_c = None if lengths is None else lengths.to(torch.int64).contiguous()
-    batch, heads, head_dim = (int(s) for s in q_c.shape)
-    seq_len = int(k_quant.original_shape[-2])
-    n_blocks = int(kv[0].shape[-3])
-    block_size = int(k_quant.block_size)
     out = torch.empty_like(q_c)
-    sm_scale = 1.0 / math.sqrt(float(head_dim))
     rows = batch * heads
-    per_channel = is_per_channel(k_quant)
-    light = q_c.dtype in (torch.float16, torch.bfloat16) and k_quant.values.dtype in (torch.int8, FP8_DTYPE)
     tiled, waves, split_tiles, max_splits, block_n = launch_plan(seq_len, rows, head_dim, block_size, block_size,
                                                                  dev, per_channel=per_channel, light=light,
                                                                  contiguous=True)
@@ -139,8 +138,8 @@ def _run_fused_dequant_attention_triton(q: torch.Tensor, k_quant: QuantizedTenso
         # split rows merge inside the decode launch (no workspace, no merge launch)
         area, area_bytes = merge_area(dev, rows, max_splits, head_dim, stream)
         _lib.check(lib.fs_fused_decode_merged(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), kv_format_code(per_channel, is_fp8(k_quant)),
-            *(t.data_ptr() for t in kv), _lib.ptr(lengths_c), out.data_ptr(), area.data_ptr(), area_bytes, batch,
+            q_c.data_ptr(), qcode, kv_format_code(per_channel, fp8),
+            *[t.data_ptr() for t in kv], _lib.ptr(lengths_c), out.data_ptr(), area.data_ptr(), area_bytes, batch,
             heads, head_dim, seq_len, n_blocks, block_size, sm_scale, split_tiles, max_splits, waves, stream))
         return _fused_result(out, return_stats, k_quant, v_quant, q_c, seq_len, max_splits, block_n, waves,
                              split_tiles, tiled)
@@ -148,15 +147,15 @@ def _run_fused_dequant_attention_triton(q: torch.Tensor, k_quant: QuantizedTenso
     if max_splits > 1:
         ws_bytes = int(lib.fs_decode_workspace_bytes(rows, max_splits, head_dim))
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    if is_fp8(k_quant):
+    if fp8:
         _lib.check(lib.fs_fused_decode_fp8(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), kv[0].data_ptr(), kv[1].data_ptr(), kv[3].data_ptr(),
+            q_c.data_ptr(), qcode, kv[0].data_ptr(), kv[1].data_ptr(), kv[3].data_ptr(),
             kv[4].data_ptr(), _lib.ptr(lengths_c), out.data_ptr(), _lib.ptr(workspace), ws_bytes, batch, heads,
             head_dim, seq_len, n_blocks, block_size, sm_scale, split_tiles, max_splits, waves, stream))
     else:
         decode = lib.fs_fused_decode_i8_channel if per_channel else lib.fs_fused_decode_i8
         _lib.check(decode(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), *(t.data_ptr() for t in kv), _lib.ptr(lengths_c),
+            q_c.data_ptr(), qcode, *[t.data_ptr() for t in kv], _lib.ptr(lengths_c),
             out.data_ptr(), _lib.ptr(workspace), ws_bytes, batch, heads, head_dim, seq_len, n_blocks, block_size,
             sm_scale, split_tiles, max_splits, waves, stream))
     if max_splits > 1:
@@ -182,17 +181,18 @@ def _fused_result(out, return_stats, k_quant, v_quant, q_c, seq_len, max_splits,
     )
 
 
+def _load_fallback():
+    from .attention import fused_dequant_attention
+
+    return fused_dequant_attention
+
+
 def fused_dequant_attention_triton(*_args: Any, **_kwargs: Any) -> Any:
     """Kernel 1 entry: HIP kernel for GPU tensors, portable ``fused_dequant_attention`` otherwise.
 
     Same signature as the reference (triton_fused.py:764-791):
     ``(q, k_quant, v_quant, lengths=None, return_stats=False)``.
     """
-
-    def _load_fallback():
-        from .attention import fused_dequant_attention
-
-        return fused_dequant_attention
 
     return dispatch_triton_or_fallback(_args, _kwargs, run_triton=_run_fused_dequant_attention_triton,
                                        load_fallback=_load_fallback)

@@ -25,7 +25,7 @@ from .triton_utils import (
     MERGE_MAX_WAVES,
     kv_format_code,
     launch_plan,
-    layout_checked,
+    layout_facts,
     merge_area,
     remember_layout,
     resolve_block_n as _resolve_block_n,
@@ -94,32 +94,35 @@ def _run_paged_quant_attention_triton(q: torch.Tensor, cache: PagedKVCache, retu
 
     kq, vq = cache.k_quant, cache.v_quant
     dev = q.device
-    table, lens = cache.block_table, cache.lengths
-    memo_key = (q.shape, q.dtype, dev, table.data_ptr(), table.numel(), lens.data_ptr(), lens.numel(),
-                kq.values.data_ptr(), kq.values.numel(), kq.scale.numel(), kq.zero_point.numel(),
-                vq.values.data_ptr(), vq.values.numel(), vq.scale.numel(), vq.zero_point.numel())
-    if not layout_checked(cache, memo_key):
+    table, lengths = cache.block_table, cache.lengths
+    kv = (kq.values, kq.scale, kq.zero_point, vq.values, vq.scale, vq.zero_point)
+    memo_key = (q.shape, q.dtype, dev, table.data_ptr(), table.numel(), lengths.data_ptr(), lengths.numel(),
+                kv[0].data_ptr(), kv[0].numel(), kv[1].numel(), kv[2].numel(),
+                kv[3].data_ptr(), kv[3].numel(), kv[4].numel(), kv[5].numel())
+    facts = layout_facts(cache, memo_key)
+    if facts is None:
         _validate_triton_paged_inputs(q, cache)
-        remember_layout(cache, memo_key)
+        batch, heads, head_dim = (int(s) for s in q.shape)
+        facts = (batch, heads, head_dim, int(kq.original_shape[0]), int(cache.block_size), int(kq.block_size),
+                 q.dtype in (torch.float16, torch.bfloat16), _lib.dtype_code(q.dtype),
+                 1.0 / math.sqrt(float(head_dim)))
+        remember_layout(cache, memo_key, facts)
+    batch, heads, head_dim, num_pages, page, quant_block, light, qcode, sm_scale = facts
+    fp8, per_channel = kv[0].dtype == FP8_DTYPE, kv[1].shape[-1] == head_dim > 1
     lib = _lib.require()
     q_c = q.contiguous()
-    kv = [t.contiguous() for t in (kq.values, kq.scale, kq.zero_point, vq.values, vq.scale, vq.zero_point)]
-    table = cache.block_table.contiguous()
-    lengths = cache.lengths if cache.lengths.dtype == torch.int64 else cache.lengths.to(torch.int64)
+    kv = [t.contiguous() for t in kv]
+    table = table.contiguous()
+    if lengths.dtype != torch.int64:
+        lengths = lengths.to(torch.int64)
     lengths = lengths.contiguous()
-    batch, heads, head_dim = (int(s) for s in q_c.shape)
     max_seq_len = int(cache.max_seq_len)
-    num_pages = int(kq.original_shape[0])
     out = torch.empty_like(q_c)
-    sm_scale = 1.0 / math.sqrt(float(head_dim))
     rows = batch * heads
-    per_channel = is_per_channel(kq)
-    light = q_c.dtype in (torch.float16, torch.bfloat16) and kq.values.dtype in (torch.int8, FP8_DTYPE)
     tiled, waves, split_tiles, max_splits, block_n = launch_plan(
-        max_seq_len, rows, head_dim, int(cache.block_size), int(kq.block_size), dev, per_channel=per_channel,
-        light=light)
+        max_seq_len, rows, head_dim, page, quant_block, dev, per_channel=per_channel, light=light)
     stream = _lib.stream_ptr(dev)
-    if request_order is not None and tiled and not per_channel and not is_fp8(kq):
+    if request_order is not None and tiled and not per_channel and not fp8:
         area, area_bytes, workspace, ws_bytes = None, 0, None, 0
         if max_splits > 1 and waves <= MERGE_MAX_WAVES:
             area, area_bytes = merge_area(dev, rows, max_splits, head_dim, stream)
@@ -127,38 +130,38 @@ def _run_paged_quant_attention_triton(q: torch.Tensor, cache: PagedKVCache, retu
             ws_bytes = int(lib.fs_decode_workspace_bytes(rows, max_splits, head_dim))
             workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         _lib.check(lib.fs_paged_decode_ordered(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), *(t.data_ptr() for t in kv), table.data_ptr(),
+            q_c.data_ptr(), qcode, *[t.data_ptr() for t in kv], table.data_ptr(),
             table.element_size(), int(table.shape[1]), lengths.data_ptr(), request_order.data_ptr(), out.data_ptr(),
             _lib.ptr(workspace), ws_bytes, _lib.ptr(area), area_bytes, batch, heads, head_dim, num_pages,
-            int(cache.block_size), int(kq.block_size), max_seq_len, sm_scale, split_tiles, max_splits, waves, stream))
+            page, quant_block, max_seq_len, sm_scale, split_tiles, max_splits, waves, stream))
         return _paged_result(out, return_stats, cache, q_c, max_seq_len, max_splits, block_n, waves, split_tiles,
                              tiled)
     if tiled and max_splits > 1 and waves <= MERGE_MAX_WAVES:
         # split rows merge inside the decode launch (no workspace, no merge launch)
         area, area_bytes = merge_area(dev, rows, max_splits, head_dim, stream)
         _lib.check(lib.fs_paged_decode_merged(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), kv_format_code(per_channel, is_fp8(kq)),
-            *(t.data_ptr() for t in kv), table.data_ptr(), table.element_size(), int(table.shape[1]),
+            q_c.data_ptr(), qcode, kv_format_code(per_channel, fp8),
+            *[t.data_ptr() for t in kv], table.data_ptr(), table.element_size(), int(table.shape[1]),
             lengths.data_ptr(), out.data_ptr(), area.data_ptr(), area_bytes, batch, heads, head_dim, num_pages,
-            int(cache.block_size), int(kq.block_size), max_seq_len, sm_scale, split_tiles, max_splits, waves, stream))
+            page, quant_block, max_seq_len, sm_scale, split_tiles, max_splits, waves, stream))
         return _paged_result(out, return_stats, cache, q_c, max_seq_len, max_splits, block_n, waves, split_tiles,
                              tiled)
     workspace, ws_bytes = None, 0
     if max_splits > 1:
         ws_bytes = int(lib.fs_decode_workspace_bytes(rows, max_splits, head_dim))
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    if is_fp8(kq):
+    if fp8:
         _lib.check(lib.fs_paged_decode_fp8(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), kv[0].data_ptr(), kv[1].data_ptr(), kv[3].data_ptr(),
+            q_c.data_ptr(), qcode, kv[0].data_ptr(), kv[1].data_ptr(), kv[3].data_ptr(),
             kv[4].data_ptr(), table.data_ptr(), table.element_size(), int(table.shape[1]), lengths.data_ptr(),
-            out.data_ptr(), _lib.ptr(workspace), ws_bytes, batch, heads, head_dim, num_pages, int(cache.block_size),
-            int(kq.block_size), max_seq_len, sm_scale, split_tiles, max_splits, waves, stream))
+            out.data_ptr(), _lib.ptr(workspace), ws_bytes, batch, heads, head_dim, num_pages, page,
+            quant_block, max_seq_len, sm_scale, split_tiles, max_splits, waves, stream))
     else:
         decode = lib.fs_paged_decode_i8_channel if per_channel else lib.fs_paged_decode_i8
         _lib.check(decode(
-            q_c.data_ptr(), _lib.dtype_code(q_c.dtype), *(t.data_ptr() for t in kv), table.data_ptr(),
+            q_c.data_ptr(), qcode, *[t.data_ptr() for t in kv], table.data_ptr(),
             table.element_size(), int(table.shape[1]), lengths.data_ptr(), out.data_ptr(), _lib.ptr(workspace),
-            ws_bytes, batch, heads, head_dim, num_pages, int(cache.block_size), int(kq.block_size), max_seq_len,
+            ws_bytes, batch, heads, head_dim, num_pages, page, quant_block, max_seq_len,
             sm_scale, split_tiles, max_splits, waves, stream))
     if max_splits > 1:
         _lib.check(lib.fs_combine_splits(
@@ -182,19 +185,21 @@ def _paged_result(out, return_stats, cache, q_c, max_seq_len, max_splits, block_
     )
 
 
+def _needs_paged_cache(args) -> bool:
+    return len(args) >= 2 and isinstance(args[1], PagedKVCache)
+
+
+def _load_fallback():
+    from .attention import paged_quant_attention
+
+    return paged_quant_attention
+
+
 def paged_quant_attention_triton(*_args: Any, **_kwargs: Any) -> Any:
     """Kernel 2 entry: HIP kernel for a GPU ``q`` with a ``PagedKVCache``, portable path otherwise.
 
     Same signature as the reference (triton_paged.py:453-490): ``(q, cache, return_stats=False)``.
     """
-
-    def _needs_paged_cache(args) -> bool:
-        return len(args) >= 2 and isinstance(args[1], PagedKVCache)
-
-    def _load_fallback():
-        from .attention import paged_quant_attention
-
-        return paged_quant_attention
 
     return dispatch_triton_or_fallback(_args, _kwargs, run_triton=_run_paged_quant_attention_triton,
                                        load_fallback=_load_fallback, extra_guard=_needs_paged_cache)

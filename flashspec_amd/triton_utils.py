@@ -14,6 +14,8 @@ import functools
 import math
 import os
 
+import torch
+
 from . import _lib
 
 HAS_HIP = _lib.available()
@@ -43,9 +45,7 @@ def dispatch_triton_or_fallback(args, kwargs, *, run_triton, load_fallback, extr
     A GPU call without the HIP library raises RuntimeError rather than falling back.
     """
 
-    import torch
-
-    if args and isinstance(args[0], torch.Tensor) and args[0].device.type == "cuda" and (
+    if args and isinstance(args[0], torch.Tensor) and args[0].is_cuda and (
         extra_guard is None or extra_guard(args)
     ):
         _lib.require()
@@ -59,18 +59,20 @@ def dispatch_triton_or_fallback(args, kwargs, *, run_triton, load_fallback, extr
 # signature (shape, dtype, device) and companions it was checked with, plus the data
 # pointers and element counts of its tensors, so repeated launches over the same cache skip
 # the checks (about 10 us of host time per call).  Any difference, including a tensor resized
-# in place, re-runs the full validation.
+# in place, re-runs the full validation.  What the launch takes from the checked shapes (its
+# ``facts``: sizes and format, no pointers) is kept with the key.
 _MEMO_ATTR = "_fs_layout_checked"
 
 
-def layout_checked(owner, key) -> bool:
-    """True when ``owner`` passed validation before with this exact ``key``."""
+def layout_facts(owner, key):
+    """The facts remembered when ``owner`` passed validation with this exact ``key``, or None."""
 
-    return owner.__dict__.get(_MEMO_ATTR) == key
+    memo = owner.__dict__.get(_MEMO_ATTR)
+    return memo[1] if memo is not None and memo[0] == key else None
 
 
-def remember_layout(owner, key) -> None:
-    object.__setattr__(owner, _MEMO_ATTR, key)
+def remember_layout(owner, key, facts) -> None:
+    object.__setattr__(owner, _MEMO_ATTR, (key, facts))
 
 
 # ---- merge areas of the in-kernel split merge -----------------------------------------------
@@ -98,8 +100,6 @@ def _merge_area_bytes(rows: int, max_splits: int, head_dim: int) -> int:
 def merge_area(device, rows: int, max_splits: int, head_dim: int, stream: int | None = None):
     """(tensor, bytes) of a zero-filled merge area for one decode launch on the current stream
     (``stream``: its handle, when the caller has it already)."""
-
-    import torch
 
     need = _merge_area_bytes(rows, max_splits, head_dim)
     if torch.cuda.is_current_stream_capturing():
@@ -222,9 +222,7 @@ _CU_CACHE: dict = {}
 
 
 def device_cu_count(device) -> int:
-    import torch
-
-    dev = torch.device(device)
+    dev = torch_device(device)
     key = dev.index if dev.index is not None else torch.cuda.current_device()
     if key not in _CU_CACHE:
         _CU_CACHE[key] = int(torch.cuda.get_device_properties(key).multi_processor_count)
@@ -436,6 +434,21 @@ def plan_tree_splits(seq_len: int, units: int, head_dim: int, cu_count: int) -> 
 _PLAN_KNOBS = ("FLASHSPEC_NUM_WARPS", "FLASHSPEC_BLOCK_N", "FLASHSPEC_NUM_SPLITS")
 
 
+def _knob_reader():
+    """A function that returns the knobs' values as they are now: os.environ's own mapping, read without
+    its per-lookup encoding where this Python has it (3 lookups: 1.2 us through os.environ.get, 0.15 us so)."""
+
+    env = os.environ
+    data, encode = getattr(env, "_data", None), getattr(env, "encodekey", None)
+    if not isinstance(data, dict) or encode is None:
+        return lambda: tuple([env.get(k) for k in _PLAN_KNOBS])
+    a, b, c = (encode(k) for k in _PLAN_KNOBS)
+    return lambda: (data.get(a), data.get(b), data.get(c))
+
+
+_knobs = _knob_reader()
+
+
 def launch_plan(seq_len: int, rows: int, head_dim: int, page_size: int, quant_block: int, device,
                 per_channel: bool = False, light: bool = False, contiguous: bool = False):
     """(tiled, waves_per_block, split_tiles, max_splits, block_n) for one decode launch.
@@ -449,15 +462,11 @@ def launch_plan(seq_len: int, rows: int, head_dim: int, page_size: int, quant_bl
     host time saved per launch)."""
 
     dev = torch_device(device)
-    env = os.environ
-    knobs = tuple(env.get(k) for k in _PLAN_KNOBS)
-    return _launch_plan_cached(int(seq_len), int(rows), int(head_dim), int(page_size), int(quant_block),
-                               dev.type, dev.index, bool(per_channel), bool(light), bool(contiguous), knobs)
+    return _launch_plan_cached(seq_len, rows, head_dim, page_size, quant_block, dev.type, dev.index, per_channel, light,
+                               contiguous, _knobs())
 
 
 def torch_device(device):
-    import torch
-
     return device if isinstance(device, torch.device) else torch.device(device)
 
 
@@ -466,10 +475,6 @@ def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, 
                         dev_index, per_channel: bool, light: bool, contiguous: bool, knobs: tuple):
     """`knobs` keys the cache and says whether any is set; the helpers below read the same values from the
     environment."""
-
-    import torch
-
-    from . import _lib
 
     device = torch.device(dev_type, dev_index) if dev_index is not None else torch.device(dev_type)
     lib = _lib.require()
