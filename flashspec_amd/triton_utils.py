@@ -261,7 +261,8 @@ def forced_tiled_waves() -> int | None:
 def plan_splits(seq_len: int, rows: int, block_n: int, cu_count: int, *, tiled: bool = True,
                 waves: int | None = None, max_waves: int = MAX_TILED_WAVES,
                 tile_group: int = 1, light: bool = False) -> tuple[int, int, int]:
-    """Return ``(split_tiles, max_splits, waves_per_block)`` for one decode launch.
+    """Return ``(split_tiles, max_splits, waves_per_block)`` for one decode launch with a knob set, or
+    of the generic kernel (``plan_rows`` plans the tiled path's other launches).
 
     ``rows`` rows of up to ``seq_len`` tokens; ``waves`` fixes the workgroup size
     (tiled path) or the waves grouped per workgroup (generic path).  ``tile_group`` > 1
