@@ -113,6 +113,9 @@ __device__ __forceinline__ void quantize_token_group(const Get& get, int rows, i
   }
 }
 
+// A launch's waves take the groups [first, groups) in order, one each (launch_ranges).
+__device__ __forceinline__ int64_t wave_in_grid() { return ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; }
+
 // Group formats of the block / page quantizers.
 enum GroupFormat : int {
   kGfAffine = 0,   // affine INT8, one scale / zero per group
@@ -543,9 +546,9 @@ struct GroupRef {
 // stores 163 us, with non-temporal ones 150.5; 32768 workgroups without a loop
 // (44 registers) 129.6, 6.2 TB/s.
 template <int GF, int CH, typename XT, typename Map>
-__device__ __forceinline__ void quantize_group_vec(const Map& map, int64_t groups, int rows, int D) {
+__device__ __forceinline__ void quantize_group_vec(const Map& map, int64_t first, int64_t groups, int rows, int D) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const int64_t grp = first + wave_in_grid();
   if (grp >= groups) return;
   const int n = rows * D;
   const LaneMap m = lane_map<GF>(n, D, lane);
@@ -579,8 +582,8 @@ __host__ __device__ constexpr int vec_chunks(int rows, int D) {
 // x [outer, S, D] -> values [outer, nb, bs, D]; groups (o, block), vectorized.
 template <int GF, int CH, typename XT>
 __global__ void __launch_bounds__(256)
-quantize_blocks_vec_kernel(const XT* x, int64_t outer, int S, int D, int bs, int nb, int8_t* values, float* scale,
-                           int16_t* zero) {
+quantize_blocks_vec_kernel(const XT* x, int64_t first, int64_t groups, int S, int D, int bs, int nb, int8_t* values,
+                           float* scale, int16_t* zero) {
   const int per = group_params<GF>(bs, D);
   auto map = [=](int64_t grp) {
     const int64_t o = grp / nb;
@@ -588,7 +591,7 @@ quantize_blocks_vec_kernel(const XT* x, int64_t outer, int S, int D, int bs, int
     return GroupRef<XT>{x + ((size_t)o * S + (size_t)blk * bs) * D, min(S - blk * bs, bs), values + (size_t)grp * bs * D,
                         scale + (size_t)grp * per, zero ? zero + (size_t)grp * per : nullptr};
   };
-  quantize_group_vec<GF, CH, XT>(map, outer * nb, bs, D);
+  quantize_group_vec<GF, CH, XT>(map, first, groups, bs, D);
 }
 
 struct PageStore {
@@ -643,10 +646,10 @@ __device__ __forceinline__ GroupRef<XT> page_group(const PagesSource<XT>& s, int
 
 template <int GF, int CH, typename XT>
 __global__ void __launch_bounds__(256)
-quantize_pages_vec_kernel(const PagesSource<XT> s, int64_t groups) {
+quantize_pages_vec_kernel(const PagesSource<XT> s, int64_t first, int64_t groups) {
   const int lane = threadIdx.x & (kWave - 1);
   auto map = [&](int64_t grp) { return page_group<GF, unsigned>(s, grp, lane); };
-  quantize_group_vec<GF, CH, XT>(map, groups, s.page, s.D);
+  quantize_group_vec<GF, CH, XT>(map, first, groups, s.page, s.D);
 }
 
 // x [outer, S, D] -> values [outer, nb, bs, D]; group = (o, block); rows past S read as 0.
@@ -654,11 +657,11 @@ quantize_pages_vec_kernel(const PagesSource<XT> s, int64_t groups) {
 // hold D entries per group.
 template <typename XT, int GF = kGfAffine>
 __global__ void __launch_bounds__(256)
-quantize_blocks_kernel(const XT* x, int64_t outer, int S, int D, int bs, int nb, int8_t* values, float* scale,
-                       int16_t* zero) {
+quantize_blocks_kernel(const XT* x, int64_t first, int64_t groups, int S, int D, int bs, int nb, int8_t* values,
+                       float* scale, int16_t* zero) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  if (grp >= outer * nb) return;
+  const int64_t grp = first + wave_in_grid();
+  if (grp >= groups) return;
   const int64_t o = grp / nb;
   const int blk = (int)(grp - o * nb);
   const XT* src = x + ((size_t)o * S) * D;
@@ -672,9 +675,9 @@ quantize_blocks_kernel(const XT* x, int64_t outer, int S, int D, int bs, int nb,
 // quantize_pages_vec_kernel for any sizes and addresses; rows past S read as 0.
 template <typename XT, int GF>
 __global__ void __launch_bounds__(256)
-quantize_pages_kernel(const PagesSource<XT> s, int64_t groups) {
+quantize_pages_kernel(const PagesSource<XT> s, int64_t first, int64_t groups) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const int64_t grp = first + wave_in_grid();
   if (grp >= groups) return;
   const GroupRef<XT> ref = page_group<GF, int64_t>(s, grp, lane);
   auto get = [&](int r, int d) -> float { return r < ref.valid_rows ? to_f32(ref.src[(size_t)r * s.D + d]) : 0.0f; };
@@ -686,11 +689,11 @@ template <typename XT>
 __global__ void __launch_bounds__(256)
 update_pages_kernel(const int8_t* in_values, const float* in_scale, const int16_t* in_zero, int64_t in_pages,
                     int in_qb, int8_t* out_values, float* out_scale, int16_t* out_zero, const int64_t* pages,
-                    const uint8_t* fresh, int64_t n_pages, const int32_t* row_src, const XT* src, int src_tokens,
-                    int H, int page, int D) {
+                    const uint8_t* fresh, int64_t first, int64_t groups, const int32_t* row_src, const XT* src,
+                    int src_tokens, int H, int page, int D) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  if (grp >= n_pages * H) return;
+  const int64_t grp = first + wave_in_grid();
+  if (grp >= groups) return;
   const int64_t i = grp / H;
   const int h = (int)(grp - i * H);
   const int64_t pg = pages ? pages[i] : i;
@@ -756,16 +759,16 @@ __device__ __forceinline__ GroupRef<XT> prompt_group(const PromptSource<XT>& s, 
 
 template <int CH, typename XT>
 __global__ void __launch_bounds__(256)
-prompt_pages_vec_kernel(const PromptSource<XT> s, int64_t groups, const PromptPages pages) {
+prompt_pages_vec_kernel(const PromptSource<XT> s, int64_t first, int64_t groups, const PromptPages pages) {
   auto map = [&](int64_t grp) { return prompt_group(s, pages, grp); };
-  quantize_group_vec<kGfAffine, CH, XT>(map, groups, s.page, s.D);
+  quantize_group_vec<kGfAffine, CH, XT>(map, first, groups, s.page, s.D);
 }
 
 template <typename XT>
 __global__ void __launch_bounds__(256)
-prompt_pages_kernel(const PromptSource<XT> s, int64_t groups, const PromptPages pages) {
+prompt_pages_kernel(const PromptSource<XT> s, int64_t first, int64_t groups, const PromptPages pages) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const int64_t grp = first + wave_in_grid();
   if (grp >= groups) return;
   const GroupRef<XT> ref = prompt_group(s, pages, grp);
   auto get = [&](int r, int d) -> float { return r < ref.valid_rows ? to_f32(ref.src[(size_t)r * s.D + d]) : 0.0f; };
@@ -978,9 +981,9 @@ __device__ __forceinline__ OT read_value(uint32_t byte, float scale, float zero)
 
 template <int RF, int W, typename OT, typename I>
 __global__ void __launch_bounds__(256)
-read_rows_kernel(const ReadParams p, int64_t units) {
+read_rows_kernel(const ReadParams p, int64_t first, int64_t units) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const int64_t wave = first + wave_in_grid();
   if (wave >= units) return;
   I t = sizeof(I) == 4 ? (I)__builtin_amdgcn_readfirstlane((int)wave) : (I)wave;
   // unit -> (tensor, b, h, page of the row, part of the page); neighbouring waves write neighbouring rows
@@ -1067,6 +1070,15 @@ read_rows_kernel(const ReadParams p, int64_t units) {
 
 static dim3 wave_grid(int64_t groups) { return dim3((unsigned)((groups + 3) / 4)); }
 
+// HIP launches fewer than 2^32 threads at a time: 2^24 - 1 workgroups of 4 waves.  go(first, grid) launches
+// one range of the groups (one wave each); all but enormous calls are a single range.
+constexpr int64_t kRangeGroups = 4 * ((1LL << 24) - 1);
+template <typename F>
+static void launch_ranges(int64_t groups, F&& go) {
+  for (int64_t first = 0; first < groups; first += kRangeGroups)
+    go(first, wave_grid(groups - first < kRangeGroups ? groups - first : kRangeGroups));
+}
+
 static bool is_pow2_chunks(int ch) { return ch == 1 || ch == 2 || ch == 4 || ch == 8; }
 
 // f(integral_constant<CH>) for the instantiated chunk counts of group_chunks.
@@ -1117,7 +1129,6 @@ static int launch_read(const char* what, ReadParams p, int sides, int rf, int ou
   if (p.unit > p.page) p.unit = p.page;
   p.per_page = (p.page + p.unit - 1) / p.unit;
   const int64_t units = (int64_t)sides * p.B * p.H * p.cols * p.per_page;
-  if ((units + 3) / 4 > 0x7fffffffLL) return set_error(FS_ERR_INVALID, std::string(what) + ": too many rows");
   const size_t esize = out_dtype == FS_F32 ? 4 : 2;
   bool four = p.D % 4 == 0;
   for (int i = 0; i < sides; ++i)
@@ -1126,10 +1137,12 @@ static int launch_read(const char* what, ReadParams p, int sides, int rf, int ou
     using OT = value_of<decltype(tag)>;
     auto go = [&](auto rf_c, auto w_c) {
       constexpr int RF = decltype(rf_c)::value, W = decltype(w_c)::value;
-      if (units <= 0x7fffffffLL)
-        hipLaunchKernelGGL((read_rows_kernel<RF, W, OT, unsigned>), wave_grid(units), dim3(256), 0, st, p, units);
-      else
-        hipLaunchKernelGGL((read_rows_kernel<RF, W, OT, int64_t>), wave_grid(units), dim3(256), 0, st, p, units);
+      launch_ranges(units, [&](int64_t first, dim3 grid) {
+        if (units <= 0x7fffffffLL)
+          hipLaunchKernelGGL((read_rows_kernel<RF, W, OT, unsigned>), grid, dim3(256), 0, st, p, first, units);
+        else
+          hipLaunchKernelGGL((read_rows_kernel<RF, W, OT, int64_t>), grid, dim3(256), 0, st, p, first, units);
+      });
     };
     auto by_width = [&](auto rf_c) {
       if (four)
@@ -1197,12 +1210,14 @@ static int launch_blocks(const char* what, const void* x, int x_dtype, int64_t o
   const bool known = by_dtype(x_dtype, [&](auto tag) {
     using XT = value_of<decltype(tag)>;
     const XT* src = (const XT*)x;
-    if (ch == 0)
-      hipLaunchKernelGGL((quantize_blocks_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
-    else
-      by_chunks(ch, [&](auto c) {
-        hipLaunchKernelGGL((quantize_blocks_vec_kernel<GF, decltype(c)::value, XT>), wave_grid(groups), dim3(256), 0, st, src, outer, S, D, bs, nb, values, scale, zero);
-      });
+    launch_ranges(groups, [&](int64_t first, dim3 grid) {
+      if (ch == 0)
+        hipLaunchKernelGGL((quantize_blocks_kernel<XT, GF>), grid, dim3(256), 0, st, src, first, groups, S, D, bs, nb, values, scale, zero);
+      else
+        by_chunks(ch, [&](auto c) {
+          hipLaunchKernelGGL((quantize_blocks_vec_kernel<GF, decltype(c)::value, XT>), grid, dim3(256), 0, st, src, first, groups, S, D, bs, nb, values, scale, zero);
+        });
+    });
   });
   return known ? check_launch(what) : set_error(FS_ERR_INVALID, std::string(what) + ": dtype code must be 0, 1 or 2");
 }
@@ -1241,12 +1256,14 @@ static int launch_pages(const char* what, const void* k, const void* v, int x_dt
     using XT = value_of<decltype(tag)>;
     const PagesSource<XT> s{(const XT*)k, (const XT*)v, ks, vs, plan.page_src, plan.table, plan.lengths, plan.P,
                             batch, H, S, D, page, nbps, plan.interleaved};
-    if (ch == 0)
-      hipLaunchKernelGGL((quantize_pages_kernel<XT, GF>), wave_grid(groups), dim3(256), 0, st, s, groups);
-    else
-      by_chunks(ch, [&](auto c) {
-        hipLaunchKernelGGL((quantize_pages_vec_kernel<GF, decltype(c)::value, XT>), wave_grid(groups), dim3(256), 0, st, s, groups);
-      });
+    launch_ranges(groups, [&](int64_t first, dim3 grid) {
+      if (ch == 0)
+        hipLaunchKernelGGL((quantize_pages_kernel<XT, GF>), grid, dim3(256), 0, st, s, first, groups);
+      else
+        by_chunks(ch, [&](auto c) {
+          hipLaunchKernelGGL((quantize_pages_vec_kernel<GF, decltype(c)::value, XT>), grid, dim3(256), 0, st, s, first, groups);
+        });
+    });
   });
   return known ? check_launch(what) : set_error(FS_ERR_INVALID, std::string(what) + ": dtype code must be 0, 1 or 2");
 }
@@ -1294,11 +1311,13 @@ extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, i
   const uintptr_t src_bits = (uintptr_t)k | (uintptr_t)v, dst_bits = (uintptr_t)k_values | (v ? (uintptr_t)v_values : 0);
   const int ch = src_bits % 16 == 0 && dst_bits % 8 == 0 ? group_chunks(page_size, head_dim, false) : 0;
   const int sides = v ? 2 : 1;
-  if ((int64_t)sides * kPromptPages * heads > 0x7fffffffLL)
-    return set_error(FS_ERR_INVALID, "write_prompt: too many (page, head) groups");
+  // pages per launch: what the arguments hold, of a group count within the kernel's 32-bit index
+  const int64_t most = 0x7fffffffLL / ((int64_t)sides * heads);
+  if (most < 1) return set_error(FS_ERR_INVALID, "write_prompt: more than 2^31 heads of K and V");
+  const int step = most < kPromptPages ? (int)most : kPromptPages;
   PromptPages ids;
-  for (int first = 0; first < n_pages; first += kPromptPages) {
-    const int n = n_pages - first < kPromptPages ? n_pages - first : kPromptPages;
+  for (int first = 0; first < n_pages; first += step) {
+    const int n = n_pages - first < step ? n_pages - first : step;
     for (int i = 0; i < n; ++i) ids.id[i] = pages[first + i];
     for (int i = n; i < kPromptPages; ++i) ids.id[i] = 0;
     const int64_t groups = (int64_t)sides * n * heads;
@@ -1306,12 +1325,14 @@ extern "C" int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, i
       using XT = value_of<decltype(tag)>;
       const PromptSource<XT> s{(const XT*)k, (const XT*)v, {k_values, k_scale, k_zero}, {v_values, v_scale, v_zero},
                                heads, src_tokens, length, head_dim, page_size, first, n};
-      if (ch == 0)
-        hipLaunchKernelGGL(prompt_pages_kernel<XT>, wave_grid(groups), dim3(256), 0, st, s, groups, ids);
-      else
-        by_chunks(ch, [&](auto c) {
-          hipLaunchKernelGGL((prompt_pages_vec_kernel<decltype(c)::value, XT>), wave_grid(groups), dim3(256), 0, st, s, groups, ids);
-        });
+      launch_ranges(groups, [&](int64_t at, dim3 grid) {
+        if (ch == 0)
+          hipLaunchKernelGGL(prompt_pages_kernel<XT>, grid, dim3(256), 0, st, s, at, groups, ids);
+        else
+          by_chunks(ch, [&](auto c) {
+            hipLaunchKernelGGL((prompt_pages_vec_kernel<decltype(c)::value, XT>), grid, dim3(256), 0, st, s, at, groups, ids);
+          });
+      });
     });
     if (!known) return set_error(FS_ERR_INVALID, "write_prompt: dtype code must be 0, 1 or 2");
     if (const int rc = check_launch("write_prompt")) return rc;
@@ -1336,13 +1357,13 @@ extern "C" int fs_update_pages_i8(const int8_t* in_values, const float* in_scale
   if (in_pages > 0 && (!in_values || !in_scale || !in_zero)) return set_error(FS_ERR_INVALID, "update_pages: null input store");
   const int64_t groups = n_pages * heads;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = wave_grid(groups), block(256);
-  switch (src_dtype) {
-    case FS_F32: hipLaunchKernelGGL(update_pages_kernel<float>, grid, block, 0, st, in_values, in_scale, in_zero, in_pages, in_quant_block, out_values, out_scale, out_zero, pages, fresh, n_pages, row_src, (const float*)src, src_tokens, heads, page_size, head_dim); break;
-    case FS_F16: hipLaunchKernelGGL(update_pages_kernel<__half>, grid, block, 0, st, in_values, in_scale, in_zero, in_pages, in_quant_block, out_values, out_scale, out_zero, pages, fresh, n_pages, row_src, (const __half*)src, src_tokens, heads, page_size, head_dim); break;
-    case FS_BF16: hipLaunchKernelGGL(update_pages_kernel<__hip_bfloat16>, grid, block, 0, st, in_values, in_scale, in_zero, in_pages, in_quant_block, out_values, out_scale, out_zero, pages, fresh, n_pages, row_src, (const __hip_bfloat16*)src, src_tokens, heads, page_size, head_dim); break;
-    default: return set_error(FS_ERR_INVALID, "update_pages: dtype code must be 0, 1 or 2");
-  }
+  const bool known = by_dtype(src_dtype, [&](auto tag) {
+    using XT = value_of<decltype(tag)>;
+    launch_ranges(groups, [&](int64_t first, dim3 grid) {
+      hipLaunchKernelGGL(update_pages_kernel<XT>, grid, dim3(256), 0, st, in_values, in_scale, in_zero, in_pages, in_quant_block, out_values, out_scale, out_zero, pages, fresh, first, groups, row_src, (const XT*)src, src_tokens, heads, page_size, head_dim);
+    });
+  });
+  if (!known) return set_error(FS_ERR_INVALID, "update_pages: dtype code must be 0, 1 or 2");
   return check_launch("update_pages");
 }
 
@@ -1364,6 +1385,7 @@ extern "C" int fs_append_tokens_i8(const void* k_new, const void* v_new, int src
     return set_error(FS_ERR_INVALID, "append_tokens: lengths_in and lengths_out must be different buffers");
   const PageStore ks{k_values, k_scale, k_zero}, vs{v_values, v_scale, v_zero};
   const int64_t groups = 2LL * batch * heads;
+  if (groups > kRangeGroups) return set_error(FS_ERR_INVALID, "append_tokens: more than 2^25 - 2 (request, head) pairs");
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid = wave_grid(groups), block(256);
   const int ch = vec_chunks(page_size, head_dim);
@@ -1399,22 +1421,23 @@ static int launch_quantize_sym(const XT* x, int64_t rows, int D, int8_t* values,
   const int lpr = D / 8;
   const bool vec = D % 8 == 0 && lpr <= kWave && (lpr & (lpr - 1)) == 0 && ((uintptr_t)x % 16) == 0 &&
                    ((uintptr_t)values % 8) == 0;
-  const dim3 block(256);
-  if (!vec) {
-    hipLaunchKernelGGL(quantize_sym_rows_generic_kernel<XT>, wave_grid(rows), block, 0, st, x, rows, D, values, scale, zero);
-    return check_launch("quantize_symmetric_per_token");
-  }
-  const int64_t waves = (rows + (kWave / lpr) - 1) / (kWave / lpr);
-  const dim3 grid = wave_grid(waves);
-  switch (lpr) {
-    case 1: hipLaunchKernelGGL((quantize_sym_rows_kernel<1, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-    case 2: hipLaunchKernelGGL((quantize_sym_rows_kernel<2, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-    case 4: hipLaunchKernelGGL((quantize_sym_rows_kernel<4, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-    case 8: hipLaunchKernelGGL((quantize_sym_rows_kernel<8, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-    case 16: hipLaunchKernelGGL((quantize_sym_rows_kernel<16, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-    case 32: hipLaunchKernelGGL((quantize_sym_rows_kernel<32, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-    default: hipLaunchKernelGGL((quantize_sym_rows_kernel<64, XT>), grid, block, 0, st, x, rows, D, values, scale, zero); break;
-  }
+  const int per_wave = vec ? kWave / lpr : 1;
+  launch_ranges((rows + per_wave - 1) / per_wave, [&](int64_t first, dim3 grid) {
+    const int64_t r0 = first * per_wave, n = rows - r0;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, x + r0 * D, n, D, values + r0 * D, scale + r0, zero + r0);
+    };
+    switch (vec ? lpr : 0) {
+      case 0: go(quantize_sym_rows_generic_kernel<XT>); break;
+      case 1: go(quantize_sym_rows_kernel<1, XT>); break;
+      case 2: go(quantize_sym_rows_kernel<2, XT>); break;
+      case 4: go(quantize_sym_rows_kernel<4, XT>); break;
+      case 8: go(quantize_sym_rows_kernel<8, XT>); break;
+      case 16: go(quantize_sym_rows_kernel<16, XT>); break;
+      case 32: go(quantize_sym_rows_kernel<32, XT>); break;
+      default: go(quantize_sym_rows_kernel<64, XT>); break;
+    }
+  });
   return check_launch("quantize_symmetric_per_token");
 }
 

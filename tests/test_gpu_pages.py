@@ -301,6 +301,77 @@ def test_dequantize_matches_the_portable_path(dtype, dim, block, seq):
         assert torch.equal(got.cpu(), want)
 
 
+# a launch holds 2^26 - 4 groups of one wave: K's 40 million end inside the first, V's pass into a second
+LAUNCH_GROUPS = 4 * (2 ** 24 - 1)
+
+
+def windows(n: int, *marks: int):
+    return [(max(0, m - 40), min(n, m + 40)) for m in (0, *marks, n)]
+
+
+@pytest.mark.parametrize("kv_format", ["affine_block", "fp8_block"])
+def test_more_groups_than_one_launch_holds(kv_format):
+    n, dim = 40_000_000, 8
+    assert n < LAUNCH_GROUPS < 2 * n
+    announce(f"from_dense and to_dense of {n} one-token pages, {kv_format}")
+    g = torch.Generator(device=DEV).manual_seed(3)
+    k, v = (torch.randn((1, 1, n, dim), generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    for x in (k, v):
+        x[..., 0] = 0  # a group's range holds 0, so that nothing is clipped
+    cache = fa.PagedKVCache.from_dense(k, v, 1, kv_format=kv_format)
+    dense = cache.to_dense()
+    quantize = fa.quantize_int8_per_block if kv_format == "affine_block" else fa.quantize_fp8_per_block
+    for name, x, q, d in (("k", k, cache.k_quant, dense[0]), ("v", v, cache.v_quant, dense[1])):
+        for a, b in windows(n, LAUNCH_GROUPS % n):
+            want = quantize(x[:, :, a:b].cpu(), 1)
+            assert torch.equal(q.values[a:b].reshape(-1, dim).cpu().view(torch.uint8),
+                               want.values.reshape(-1, dim).view(torch.uint8)), (name, a)
+            assert torch.equal(q.scale[a:b].reshape(-1).cpu(), want.scale.reshape(-1)), (name, a)
+            assert torch.equal(d[:, :, a:b].cpu(), fa.dequantize_int8_per_block(want)), (name, a)
+        # every page of both ranges was written and read: FP8 is off by at most 448 / 16 scales, INT8 by one (half
+        # by rounding, half where the rounded zero point clips an end)
+        step = q.scale.reshape(1, 1, n, 1) * (32.0 if kv_format == "fp8_block" else 1.01)
+        assert bool(((d - x.float()).abs() <= step).all()), name
+    ids = torch.arange(n, device=DEV)
+    assert torch.equal(cache.block_table.reshape(-1), ids)
+
+
+def test_block_quantizer_of_more_groups_than_one_launch_holds():
+    n, dim = LAUNCH_GROUPS + 5, 8
+    announce(f"quantize_int8_per_block of {n} one-token blocks")
+    x = torch.randn((n, dim), generator=torch.Generator(device=DEV).manual_seed(4), device=DEV, dtype=torch.float16)
+    x[:, 0] = 0  # as above
+    q = fa.quantize_int8_per_block(x, 1)
+    back = fa.dequantize_int8_per_block(q, dtype=torch.float16)
+    for a, b in windows(n, LAUNCH_GROUPS):
+        want = fa.quantize_int8_per_block(x[a:b].cpu(), 1)
+        assert torch.equal(q.values[a:b].cpu(), want.values) and torch.equal(q.scale[a:b].cpu(), want.scale), a
+        assert torch.equal(back[a:b].cpu(), fa.dequantize_int8_per_block(want, dtype=torch.float16)), a
+    # one step of the block plus the half-precision rounding of a value under 8 (2^-9 of it at most)
+    assert bool(((back - x).abs().float() <= 1.01 * q.scale.reshape(n, 1) + 2.0 ** -8).all())
+    announce(f"fs_update_pages_i8 of {n} one-token pages")
+    out = [torch.empty_like(t) for t in (q.values, q.scale, q.zero_point)]
+    rows = torch.arange(n, dtype=torch.int32, device=DEV)
+    _lib.check(_lib.require().fs_update_pages_i8(
+        None, None, None, 0, 1, *(t.data_ptr() for t in out), None, None, n, rows.data_ptr(), x.data_ptr(),
+        _lib.dtype_code(x.dtype), n, 1, 1, dim, _lib.stream_ptr(DEV)))
+    for got, want in zip(out, (q.values, q.scale, q.zero_point)):
+        assert torch.equal(got, want)
+
+
+def test_token_quantizer_of_more_rows_than_one_launch_holds():
+    n, dim = LAUNCH_GROUPS + 5, 4  # a wave per row
+    announce(f"quantize_int8_symmetric_per_token of {n} rows")
+    x = torch.randn((n, dim), generator=torch.Generator(device=DEV).manual_seed(5), device=DEV, dtype=torch.float16)
+    q = fa.quantize_int8_symmetric_per_token(x)
+    for a, b in windows(n, LAUNCH_GROUPS):
+        want = fa.quantize_int8_symmetric_per_token(x[a:b].cpu())
+        assert torch.equal(q.values[a:b].cpu(), want.values) and torch.equal(q.scale[a:b].cpu(), want.scale), a
+    back = q.values.reshape(n, dim) * q.scale.reshape(n, 1)
+    assert bool(((back - x.float()).abs() <= 0.51 * q.scale.reshape(n, 1)).all())
+    assert bool((q.zero_point == 128).all())
+
+
 def test_prompt_entry_rejects_bad_sizes():
     lib = _lib.require()
     ids = (np.zeros(4, dtype=np.int32)).ctypes.data
