@@ -261,8 +261,8 @@ def forced_tiled_waves() -> int | None:
 def plan_splits(seq_len: int, rows: int, block_n: int, cu_count: int, *, tiled: bool = True,
                 waves: int | None = None, max_waves: int = MAX_TILED_WAVES,
                 tile_group: int = 1, light: bool = False) -> tuple[int, int, int]:
-    """Return ``(split_tiles, max_splits, waves_per_block)`` for one decode launch with a knob set, or
-    of the generic kernel (``plan_rows`` plans the tiled path's other launches).
+    """Return ``(split_tiles, max_splits, waves_per_block)`` for one decode launch whose split count or
+    wave count a knob forces, or of the generic kernel (``plan_rows`` plans the tiled path's other launches).
 
     ``rows`` rows of up to ``seq_len`` tokens; ``waves`` fixes the workgroup size
     (tiled path) or the waves grouped per workgroup (generic path).  ``tile_group`` > 1
@@ -474,8 +474,7 @@ def torch_device(device):
 @functools.lru_cache(maxsize=512)
 def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, quant_block: int, dev_type: str,
                         dev_index, per_channel: bool, light: bool, contiguous: bool, knobs: tuple):
-    """`knobs` keys the cache and says whether any is set; the helpers below read the same values from the
-    environment."""
+    """`knobs` only keys the cache: the helpers below read the same values from the environment."""
 
     device = torch.device(dev_type, dev_index) if dev_index is not None else torch.device(dev_type)
     lib = _lib.require()
@@ -495,7 +494,9 @@ def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, 
     # the default plan's ceiling (a forced wave count keeps only the register limit above)
     if contiguous and tiled and not per_channel and head_dim == 64:
         max_waves = min(max_waves, CONTIGUOUS_D64_WAVES)
-    if tiled and not any(knobs):
+    # by what the knobs force: FLASHSPEC_BLOCK_N alone (it only clamps a forced split count) and values
+    # that are no valid setting leave the default plan
+    if tiled and waves is None and forced_num_splits(seq_len, block_n) is None:
         split_tiles, max_splits, waves = plan_rows(seq_len, rows, head_dim, device_cu_count(device),
                                                    max_waves=max_waves, tile_group=group, light=light,
                                                    per_channel=per_channel)

@@ -5,7 +5,9 @@ from __future__ import annotations
 import math
 
 import pytest
+import torch
 
+from flashspec_amd import triton_utils
 from flashspec_amd.triton_utils import plan_rows
 
 
@@ -35,3 +37,41 @@ def test_plans_at_the_lines_of_the_rule():
     assert plan(4096, 256) == (256, 1, 16) and plan(4096, 256, light=True) == (256, 1, 4)
     assert plan(2032, 512) == (127, 1, 8) and plan(2048, 512) == (128, 1, 16)
     assert plan(512, 64, 256, max_waves=8) == (16, 2, 4) and plan(512, 64) == (32, 1, 8)
+
+
+@pytest.fixture()
+def launch_plan(monkeypatch):
+    """triton_utils.launch_plan for a GPU of 256 CUs with no knob set, and a setter of knobs."""
+
+    from flashspec_amd import _lib
+
+    _lib.require()  # the tiled-path rule is a host function of the library
+    for key in triton_utils._PLAN_KNOBS:
+        monkeypatch.delenv(key, raising=False)
+    monkeypatch.setitem(triton_utils._CU_CACHE, 0, 256)
+    triton_utils._launch_plan_cached.cache_clear()
+    yield (lambda seq, rows, dim=128, **kw: triton_utils.launch_plan(seq, rows, dim, 16, 16, torch.device("cuda", 0), **kw),
+           monkeypatch.setenv)
+    triton_utils._launch_plan_cached.cache_clear()
+
+
+@pytest.mark.parametrize("knob,value", [
+    ("FLASHSPEC_BLOCK_N", "128"), ("FLASHSPEC_BLOCK_N", "16"), ("FLASHSPEC_BLOCK_N", "48"), ("FLASHSPEC_BLOCK_N", ""),
+    ("FLASHSPEC_NUM_SPLITS", "0"), ("FLASHSPEC_NUM_SPLITS", "-1"), ("FLASHSPEC_NUM_SPLITS", "many"),
+    ("FLASHSPEC_NUM_WARPS", "3"), ("FLASHSPEC_NUM_WARPS", "x")])
+def test_knobs_that_force_nothing_leave_the_default_plan(launch_plan, knob, value):
+    plan, setenv = launch_plan
+    shapes = [(seq, rows, dim, light) for seq in (128, 1024, 4096, 16384) for rows in (8, 96, 128, 160, 256, 512)
+              for dim in (64, 128, 256) for light in (False, True)]
+    default = [plan(seq, rows, dim, light=light)[:4] for seq, rows, dim, light in shapes]
+    setenv(knob, value)
+    assert [plan(seq, rows, dim, light=light)[:4] for seq, rows, dim, light in shapes] == default
+
+
+def test_knobs_that_force_a_plan_still_do(launch_plan):
+    plan, setenv = launch_plan
+    assert plan(4096, 96)[1:4] == (8, 128, 2)
+    setenv("FLASHSPEC_NUM_WARPS", "4")
+    assert plan(4096, 96)[1] == 4
+    setenv("FLASHSPEC_NUM_SPLITS", "4")
+    assert plan(4096, 96)[1:4] == (4, 64, 4)
