@@ -15,7 +15,7 @@ free list, tables, lengths — stays in Python like the reference's.
 from __future__ import annotations
 
 from array import array
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import Dict, Sequence, Tuple
 
 import numpy as np
@@ -413,6 +413,8 @@ class PagedKVCache:
     ``k_quant/v_quant`` hold the physical store (``original_shape = [P, H, page, D]``),
     ``block_table [batch, cols]`` maps logical to physical pages (-1 = unallocated),
     ``lengths [batch]`` the valid tokens per row, ``max_seq_len`` the attention span.
+    ``full_rows`` tells the launch planner that the rows were (nearly) full when the cache was built; no
+    result depends on it.
     """
 
     k_quant: QuantizedTensor
@@ -421,6 +423,7 @@ class PagedKVCache:
     lengths: torch.Tensor
     block_size: int
     max_seq_len: int
+    full_rows: bool = field(default=False, kw_only=True, compare=False)
 
     @property
     def batch_size(self) -> int:
@@ -472,13 +475,15 @@ class PagedKVCache:
         if not on_gpu or pattern in {"shuffled", "random"}:
             perm = _layout_permutation(pattern, batch, blocks_per_seq, layout_seed, k.device)
 
-        effective_lengths = None
+        effective_lengths, full_rows = None, True
         if lengths is not None:
             effective_lengths = lengths.to(device=k.device, dtype=torch.int64).contiguous()
             if effective_lengths.ndim != 1 or effective_lengths.shape[0] != batch:
                 raise ValueError("lengths must be [batch]")
-            if bool((effective_lengths < 0).any().item()) or bool((effective_lengths > seq_len).any().item()):
+            held = effective_lengths.tolist()
+            if any(not 0 <= n <= seq_len for n in held):
                 raise ValueError("lengths must lie in [0, seq_len]")
+            full_rows = 4 * sum(held) >= 3 * batch * seq_len
 
         if on_gpu:
             k_quant, v_quant, block_table, full_lengths = cls._build_hip(k, v, block_size, perm,
@@ -503,7 +508,7 @@ class PagedKVCache:
                             "affine_channel": quantize_int8_per_channel}[kv_format]
                 k_quant, v_quant = quantize(k_pages, block_size=block_size), quantize(v_pages, block_size=block_size)
         return cls(k_quant=k_quant, v_quant=v_quant, block_table=block_table, lengths=effective_lengths,
-                   block_size=block_size, max_seq_len=seq_len)
+                   block_size=block_size, max_seq_len=seq_len, full_rows=full_rows)
 
     @staticmethod
     def _physical_pages(x: torch.Tensor, block_size: int, perm: torch.Tensor | None) -> torch.Tensor:

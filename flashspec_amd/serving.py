@@ -453,8 +453,9 @@ class DecodeBatch:
         # every row covers its appended token: the longest request after the step, in whole pages
         max_seq_len = -(-(max(self.host_lengths) + 1) // self.page) * self.page
         rows = len(self._requests) * a.heads
+        # as for full rows: a plan of one round of workgroups, which is what one launch can run
         plan = launch_plan(max_seq_len, rows, a.head_dim, self.page, self.page, self.device,
-                           light=q.dtype in (torch.float16, torch.bfloat16))
+                           light=q.dtype in (torch.float16, torch.bfloat16), full_rows=True)
         if rows * plan[3] > device_cu_count(self.device):
             return None
         return max_seq_len, plan

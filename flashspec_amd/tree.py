@@ -133,7 +133,8 @@ def _hip(q, cache, draft_k, draft_v, parents_dev, dims, kernel):
     else:
         tiled, waves, split_tiles, max_splits, block_n = launch_plan(max_seq_len, rows, head_dim,
                                                                      int(cache.block_size), int(kq.block_size), dev,
-                                                                     per_channel=per_channel)
+                                                                     per_channel=per_channel,
+                                                                     full_rows=cache.full_rows)
     out = torch.empty_like(q_c)
     stream = _lib.stream_ptr(dev)
     plan = {"num_splits": float(max_splits), "split_tiles": float(split_tiles), "num_warps": float(waves),

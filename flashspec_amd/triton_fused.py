@@ -44,7 +44,7 @@ def _compute_num_splits(seq_len: int, block_n: int) -> int:
 
     ``FLASHSPEC_NUM_SPLITS`` wins (clamped to ``ceil(seq_len/block_n)``); otherwise
     1 split up to 512 tokens, else ``min(4, ceil(seq_len/block_n))`` capped at 32.
-    The HIP launch sizes its splits for the GPU instead (``triton_utils.plan_splits``)
+    The HIP launch sizes its splits for the GPU instead (``triton_utils.launch_plan``)
     and honours the same environment override.
     """
 
@@ -132,7 +132,7 @@ def _run_fused_dequant_attention_triton(q: torch.Tensor, k_quant: QuantizedTenso
     rows = batch * heads
     tiled, waves, split_tiles, max_splits, block_n = launch_plan(seq_len, rows, head_dim, block_size, block_size,
                                                                  dev, per_channel=per_channel, light=light,
-                                                                 contiguous=True)
+                                                                 contiguous=True, full_rows=lengths is None)
     stream = _lib.stream_ptr(dev)
     if tiled and max_splits > 1 and waves <= MERGE_MAX_WAVES:
         # split rows merge inside the decode launch (no workspace, no merge launch)

@@ -120,7 +120,8 @@ def _run_paged_quant_attention_triton(q: torch.Tensor, cache: PagedKVCache, retu
     out = torch.empty_like(q_c)
     rows = batch * heads
     tiled, waves, split_tiles, max_splits, block_n = launch_plan(
-        max_seq_len, rows, head_dim, page, quant_block, dev, per_channel=per_channel, light=light)
+        max_seq_len, rows, head_dim, page, quant_block, dev, per_channel=per_channel, light=light,
+        full_rows=cache.full_rows)
     stream = _lib.stream_ptr(dev)
     if request_order is not None and tiled and not per_channel and not fp8:
         area, area_bytes, workspace, ws_bytes = None, 0, None, 0

@@ -157,20 +157,21 @@ def resolve_num_warps() -> int:
 
 
 # ---- split-K planning for the HIP kernels ---------------------------------------------------
-# Tiled path: one split = one workgroup of W cooperating waves.  Rows split only when
-# there are fewer rows than CUs (the split count fills the GPU, each split keeping at
-# least MIN_SPLIT_TILES tiles); W is then the largest power of two up to 16 that leaves
-# every wave MIN_TILES_PER_WAVE tiles, unless FLASHSPEC_NUM_WARPS fixes it.  A split
-# holds at most 64 tiles per wave.  Generic path: one split = one wave of 8..64 tiles.
+# Tiled path: one split = one workgroup of W cooperating waves, at most 64 tiles a wave.  plan_rows (below)
+# plans launches whose counts no knob forces.  plan_splits serves the others: FLASHSPEC_NUM_SPLITS fixes the
+# split count; with FLASHSPEC_NUM_WARPS alone rows split when there are fewer rows than CUs (the split count
+# fills the GPU, each split keeping at least MIN_SPLIT_TILES tiles).  W is then the largest power of two up
+# to 16 that leaves every wave MIN_TILES_PER_WAVE tiles, unless FLASHSPEC_NUM_WARPS fixes it.
+# Generic path: one split = one wave of 8..64 tiles.
 MAX_TILED_WAVES = 16
 MIN_SPLIT_TILES = 8
 MIN_TILES_PER_WAVE = 4
 MAX_TILES_PER_WAVE = 64
 # Light tiles (fp16 or bf16 query, INT8 or FP8 E4M3 values with one scale (and zero point) per
 # 16-token page, head_dim 128: the fp16 dot2 score path with every lane busy; bf16 rows enter it
-# scaled by a power of two) run 4-wave workgroups when the grid puts one workgroup on 3/4 to all of
-# the CUs and a split holds 128..256 tiles (32..64 per wave, so no extra split).  Measured on MI355X
-# (one box each, settled clocks, 3 rotated input sets), paged / fused us with 4 against 16 waves:
+# scaled by a power of two) run 4-wave workgroups when the grid puts one workgroup on all of the CUs
+# (plan_splits: on 3/4 to all of them) and a split holds 64..256 tiles (16..64 per wave, so no extra split).
+# Measured on MI355X (one box each, settled clocks, 3 rotated input sets), paged / fused us with 4 against 16 waves:
 # B8 H32 S4096 D128 43.4 / 42.1 vs 45.5 / 43.1 (bf16 query: 41.6-41.7 / 41.0-41.1 vs 44.2 /
 # 42.9-43.8; FP8 values: 43.5-44.2 / 40.9-41.1 vs 44.1-44.3 / 44.2-44.4), S2048 25.1 / 24.3 vs
 # 26.4 / 24.8, B4 S8192 46.4 / 45.0 vs 49.0 / 46.3, B2 S8192 29.3 / 27.3 vs 30.1 / 27.8, B1 S16384
@@ -185,8 +186,8 @@ MAX_TILES_PER_WAVE = 64
 # merge launch; B2 S4096 4 x 4 merged 17.52 against 20.62 for 4 x 16 with the merge launch.
 LIGHT_WAVES = 4
 LIGHT_MIN_SPLIT_TILES = 64
-# Rows that fill at least half of the CUs split in two only when each half keeps 128 tiles (light
-# tiles: LIGHT_MIN_SPLIT_TILES); otherwise they run unsplit with at most 8 waves per workgroup.
+# plan_splits with a forced wave count: rows that fill at least half of the CUs split in two only when each
+# half keeps 128 tiles (light tiles: LIGHT_MIN_SPLIT_TILES); otherwise they run unsplit.
 # Measured on MI355X before the in-kernel merge, B4 H32 S2048 D128 (fp16 query), paged / fused us:
 # unsplit x 8 waves 18.2 / 17.6, unsplit x 16 19.3 / 18.0, 2 splits x 16 19.1 / 18.4;
 # B4 S4096 (256 tiles) keeps its split: 2 x 4 waves 29.1 / 27.9 against unsplit x 8 29.9 / 29.3.
@@ -320,59 +321,92 @@ def plan_splits(seq_len: int, rows: int, block_n: int, cu_count: int, *, tiled: 
     return split_tiles, math.ceil(tiles / split_tiles), waves
 
 
-# The default plan of the tiled path (no knob set; plan_splits serves the knobs).  Measured on MI355X
-# over 5 KV formats and head_dims, 8 to 384 rows of 16 to 1024 tiles, every split count and 4 / 8 / 16
-# waves (kernel time, us):
-# * Splits never put more workgroups than CUs: a second, nearly empty round costs a whole split.
-#   B5 H32 S4096 D128 (160 rows): 2 splits 41.0, unsplit 29.8; B3 (96 rows): 3 splits 30.3, 2 splits 20.6.
-# * Rows on over half of the CUs but not all take splits of 4 waves from PLAN_SLOT_TILES on, two
-#   workgroups a CU: rows of unlike length then spread (160 rows of up to 313 tiles, per-channel: whole
-#   62.9, 2 splits of 8 waves 48.2; 160 full rows of 256 tiles: 56.0, 61.2 and, 3 of 4 waves, 43.8).
-# * A row takes at most sqrt(tiles) / 2 splits: the last split's merge grows with their number.  8 rows
-#   of 1024 tiles: 32 splits 20.6, 16 splits 16.3; 8 rows of 128 tiles: 16 splits 11.4, 4 splits 8.5.
+# The default plan of the tiled path (plan_splits serves forced counts).  Measured on MI355X, kernel time of
+# paged launches in us, 7 formats (INT8 with fp16 or fp32 queries, FP8, per-token, per-channel, head_dim 64
+# and 256), 1 to 640 rows of 8 to 1024 tiles, every row full or rows of unlike length ("ragged"; the figures
+# are the mean of 4 draws), splits x waves.  Figures are INT8, fp16 queries, 128 dims where no format is
+# named.
+# * A row takes at most sqrt(tiles) / 2 splits: the last split's merge grows with their number.  4 rows of
+#   1024 tiles: 64 splits 29.0, 16 splits 16.0; 8 rows of 128 tiles: 16 splits 12.1, 5 splits 9.3.
 # * Rows under PLAN_MIN_TILES stay whole (64 rows of 32 tiles: 4 splits 7.8, unsplit 6.6); 256-dim and
 #   per-channel tiles, whose tiles cost about twice as much, from half of that.
-# * 8 waves per workgroup, two tiles a wave at least (four at 256 dims or with more rows than CUs),
-#   merged in the launch: splits on 16 waves paid a workspace and a merge launch (B2 S8192 per-token
-#   27.4, on 8 waves 25.2).
-# * Light tiles (LIGHT_WAVES) take 4 waves where a workgroup lands on nearly every CU and a wave keeps
-#   16 to 64 tiles (256 rows of 256 tiles: 42.1, on 8 waves 44.2; 224 rows: 39.9 and 38.6).
-# * As many rows as CUs or more: 8 waves, and 16 from PLAN_LONG_TILES on, where rows of unlike length
-#   leave the last round to few workgroups (512 rows of 64 tiles: 24.1, on 16 waves 26.6; of up to 188 tiles,
+# * One round: splits that leave no workgroup for a second round, which costs a whole split (96 full rows of
+#   256 tiles: 3 x 16 32.1, 2 x 8 20.7).  8 waves per workgroup, two tiles a wave at least (four at 256 dims
+#   or with more rows than CUs), merged in the launch; 16 waves and a merge launch only where a wave of 8
+#   would hold 64 tiles (128 rows of 1024 tiles: 2 x 8 99.8, 2 x 16 89.5).
+# * That leaves CUs idle where rows do not divide them.  Whole rows on over half of the CUs take two
+#   workgroups a CU from PLAN_SLOT_TILES on: three 4-wave splits (144 rows of 256 tiles: 1 x 16 30.3, 3 x 4
+#   30.5, ragged 27.9 and 23.6), or two below PLAN_WHOLE_TILES (224 rows of 256: 1 x 8 41.4, 2 x 4 42.4; 240
+#   ragged: 34.8 and 31.9).  From there on two 4-wave splits lose to the whole row on 16 waves (240 rows of
+#   512 tiles: 106.1 and 79.6), and costly tiles gain nothing from them at all (256 dims, 192 rows of 256: 2
+#   x 4 78.7, 1 x 8 63.8).
+# * Ragged rows leave some of their splits empty, so that a few workgroups too many cost them nothing
+#   (full_rows: the host knows that every row holds seq_len tokens).  One split more: per-channel tiles, 96
+#   rows of 512 (full 2 x 8 59.7, 3 x 8 79.5; ragged 56.3 and 46.1) and 52 rows (ragged 4 x 8 32.4, 5 x 8
+#   28.5), 256 dims where it is 4% over the CUs (88 rows of 256 tiles, ragged: 27.7 and 23.0).  Four splits
+#   in place of three gain nothing (80 rows, per-channel, 256 tiles, ragged: 3 x 8 24.8, 4 x 8 29.1).  Other
+#   tiles, two splits too few: two workgroups a CU from PLAN_WHOLE_TILES on (96 ragged rows of 512: 2 x 8
+#   30.5, 5 x 4 27.8), three splits of 16 waves from PLAN_DEEP_TILES (96 ragged rows of 1024: 2 x 8 53.0, 3
+#   x 16 44.9; not the 64-dim layout).
+# * Light tiles (LIGHT_WAVES) take 4 waves where a workgroup lands on every CU and a wave keeps 16 to 64
+#   tiles (256 rows of 256 tiles: 42.1, on 8 waves 44.2), and with full rows on nearly every CU (48 rows of
+#   768: 5 x 4 29.4, 5 x 8 32.1; 120 ragged rows of 512 instead: 2 x 4 40.1, 2 x 8 31.6).
+# * As many rows as CUs or more: 8 waves, and 16 from PLAN_LONG_TILES on, where rows of unlike length leave
+#   the last round to few workgroups (512 rows of 64 tiles: 24.1, on 16 waves 26.6; of up to 188 tiles,
 #   falling to 1/16: 41.5 and 38.2).
 PLAN_MIN_TILES = 64
+PLAN_RAGGED_TILES = 96
 PLAN_LONG_TILES = 128
 PLAN_SLOT_TILES = 256
+PLAN_WHOLE_TILES = 512
+PLAN_DEEP_TILES = 768
 PLAN_WAVES = 8
-PLAN_LIGHT_MIN_FILL = 0.9
+PLAN_LIGHT_FILL = 0.97
+PLAN_LIGHT_FULL_ROWS_FILL = 0.9
 
 
 def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_waves: int = MAX_TILED_WAVES,
-              tile_group: int = 1, light: bool = False, per_channel: bool = False) -> tuple[int, int, int]:
+              tile_group: int = 1, light: bool = False, per_channel: bool = False,
+              full_rows: bool = False) -> tuple[int, int, int]:
     """``(split_tiles, max_splits, waves_per_block)`` of a tiled decode launch (rule above); arguments as
-    for ``plan_splits``."""
+    for ``plan_splits``.  ``full_rows``: as far as the host knows, every row holds ``seq_len`` tokens."""
 
     tiles = max(1, math.ceil(seq_len / TILE_TOKENS))
     grp = max(1, tile_group)
     groups = math.ceil(tiles / grp)
     costly = head_dim > 128 or per_channel
+    one_round = cu_count // max(1, rows)
     n = 1
     if tiles >= (PLAN_MIN_TILES // 2 if costly else PLAN_MIN_TILES):
-        n = max(1, min(cu_count // max(1, rows), int(math.sqrt(tiles) / 2), groups))
-    paired = n == 1 and cu_count < 2 * rows < 2 * cu_count and tiles >= PLAN_SLOT_TILES
-    if paired:
-        n = min(2 * cu_count // rows, groups)
+        n = max(1, min(one_round, int(math.sqrt(tiles) / 2), groups))
+    side_by_side = deep = False  # two smaller workgroups a CU; splits of 16 waves with a merge launch
+    if n == one_round and n * rows < cu_count:
+        pairs = 2 * cu_count // rows
+        if costly and not full_rows and _ragged_costly_split(n, tiles, (n + 1) * rows / cu_count, per_channel):
+            n += 1
+        elif n == 1 and tiles >= PLAN_SLOT_TILES:
+            side_by_side = pairs == 3 or (not costly and tiles < PLAN_WHOLE_TILES)
+        elif n == 2 and not costly and not full_rows:
+            deep = tiles >= PLAN_DEEP_TILES and head_dim > 64 and 9 * rows <= 4 * cu_count
+            side_by_side = not deep and tiles >= PLAN_WHOLE_TILES and pairs > 4
+        n = min(pairs if side_by_side else (n + 1 if deep else n), groups)
     split_groups = math.ceil(groups / n)
     n = math.ceil(groups / split_groups)
     split = split_groups * grp
-    per_wave = max(4 if head_dim > 128 or rows > cu_count else 2, grp)
+    fill = rows * n / cu_count
+    every_cu = light and grp == 1 and PLAN_LIGHT_FILL < fill <= 1
+    nearly_every_cu = light and grp == 1 and full_rows and PLAN_LIGHT_FULL_ROWS_FILL < fill <= 1
+    # light tiles on every CU keep four a wave (256 rows of 16 tiles: on 4 waves 6.5, on 8 waves 7.0)
+    per_wave = max(4 if head_dim > 128 or rows > cu_count or (every_cu and tiles >= 16) else 2, grp)
     waves = 1
     while waves < min(PLAN_WAVES, max_waves) and 2 * waves * per_wave <= split:
         waves *= 2
-    if paired or (light and grp == 1 and PLAN_LIGHT_MIN_FILL * cu_count < rows * n <= cu_count and
-                 LIGHT_MIN_SPLIT_TILES <= split <= LIGHT_WAVES * MAX_TILES_PER_WAVE):
+    if side_by_side:  # the 64-dim layout's tiles are half as long: ragged 144 rows of 512, 3 x 4 27.9, 3 x 8 25.0
+        waves = min(waves, PLAN_WAVES if head_dim <= 64 and not full_rows else LIGHT_WAVES)
+    elif split >= LIGHT_MIN_SPLIT_TILES and (every_cu and split <= LIGHT_WAVES * MAX_TILES_PER_WAVE or
+                                             nearly_every_cu and split < LIGHT_WAVES * MAX_TILES_PER_WAVE):
         waves = min(waves, LIGHT_WAVES)
-    elif rows >= cu_count and split >= PLAN_LONG_TILES:
+    elif deep or split >= PLAN_WHOLE_TILES or (rows >= cu_count and split >= PLAN_LONG_TILES):
         waves = max_waves
     while waves < max_waves and split_groups > MAX_TILES_PER_WAVE // grp * waves:
         waves *= 2
@@ -380,6 +414,15 @@ def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_wave
     if split_groups > cap:
         split_groups = math.ceil(groups / math.ceil(groups / cap))
     return split_groups * grp, math.ceil(tiles / (split_groups * grp)), waves
+
+
+def _ragged_costly_split(n: int, tiles: int, over: float, per_channel: bool) -> bool:
+    """Whether ragged rows of costly tiles take a split more than the ``n`` of one round, which asks for
+    ``over`` times the CUs (rule above)."""
+
+    if not per_channel:
+        return n == 2 and tiles >= PLAN_RAGGED_TILES and over <= 1.04
+    return (n == 2 and tiles >= PLAN_RAGGED_TILES) or (n != 3 and tiles >= 2 * PLAN_RAGGED_TILES and over <= 1.13)
 
 
 # One 8-wave workgroup of the multi-query kernel holds a CU (its ~140 registers per lane leave
@@ -451,12 +494,13 @@ _knobs = _knob_reader()
 
 
 def launch_plan(seq_len: int, rows: int, head_dim: int, page_size: int, quant_block: int, device,
-                per_channel: bool = False, light: bool = False, contiguous: bool = False):
+                per_channel: bool = False, light: bool = False, contiguous: bool = False, full_rows: bool = False):
     """(tiled, waves_per_block, split_tiles, max_splits, block_n) for one decode launch.
 
     ``light``: fp16 or bf16 query over INT8 or FP8 values (the caller's part of the LIGHT_WAVES condition;
     the store layout part is checked here).  ``contiguous``: rows of a contiguous store (the fused
-    kernel), whose default plan at head_dim 64 takes at most CONTIGUOUS_D64_WAVES waves.
+    kernel), whose default plan at head_dim 64 takes at most CONTIGUOUS_D64_WAVES waves.  ``full_rows``: see
+    ``plan_rows``.
 
     The plan is a pure function of the shape, the device and the three env knobs, which are
     read on every call; it is computed once per distinct combination (a few microseconds of
@@ -464,7 +508,7 @@ def launch_plan(seq_len: int, rows: int, head_dim: int, page_size: int, quant_bl
 
     dev = torch_device(device)
     return _launch_plan_cached(seq_len, rows, head_dim, page_size, quant_block, dev.type, dev.index, per_channel, light,
-                               contiguous, _knobs())
+                               contiguous, full_rows, _knobs())
 
 
 def torch_device(device):
@@ -473,7 +517,7 @@ def torch_device(device):
 
 @functools.lru_cache(maxsize=512)
 def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, quant_block: int, dev_type: str,
-                        dev_index, per_channel: bool, light: bool, contiguous: bool, knobs: tuple):
+                        dev_index, per_channel: bool, light: bool, contiguous: bool, full_rows: bool, knobs: tuple):
     """`knobs` only keys the cache: the helpers below read the same values from the environment."""
 
     device = torch.device(dev_type, dev_index) if dev_index is not None else torch.device(dev_type)
@@ -499,7 +543,7 @@ def _launch_plan_cached(seq_len: int, rows: int, head_dim: int, page_size: int, 
     if tiled and waves is None and forced_num_splits(seq_len, block_n) is None:
         split_tiles, max_splits, waves = plan_rows(seq_len, rows, head_dim, device_cu_count(device),
                                                    max_waves=max_waves, tile_group=group, light=light,
-                                                   per_channel=per_channel)
+                                                   per_channel=per_channel, full_rows=full_rows)
     else:
         split_tiles, max_splits, waves = plan_splits(seq_len, rows, block_n, device_cu_count(device), tiled=tiled,
                                                      waves=waves, max_waves=max_waves, tile_group=group, light=light)

@@ -8,6 +8,7 @@ graph capture with replays."""
 
 from __future__ import annotations
 
+import dataclasses
 import math
 
 import numpy as np
@@ -234,3 +235,39 @@ def test_stale_merge_words_from_earlier_launches_are_not_taken(monkeypatch):
     finally:
         area.zero_()
         torch.cuda.synchronize(DEV)
+
+
+# one call on each side of the default plan's lines for rows that leave CUs idle: a split more than one
+# round holds, two workgroups a CU, 16-wave splits (merge launch), whole rows
+@pytest.mark.parametrize("batch,heads,seq,dim,kv_format,ragged_plan,full_plan", [
+    (11, 8, 12288, 128, "affine_block", (3, 16), (2, 8)),
+    (12, 8, 8192, 128, "fp8_block", (5, 4), (2, 8)),
+    (12, 8, 8192, 64, "affine_block", (5, 8), (2, 8)),
+    (12, 8, 1536, 128, "affine_channel", (3, 8), (2, 8)),
+    (11, 8, 1536, 256, "affine_block", (3, 8), (2, 8)),
+    (6, 8, 4090, 128, "affine_channel", (6, 8), (5, 8)),
+    (18, 8, 4096, 64, "symmetric_token", (3, 8), (3, 4)),
+    (24, 8, 8192, 128, "affine_block", (1, 16), (1, 16)),
+])
+def test_default_plans_of_rows_that_leave_cus_idle(batch, heads, seq, dim, kv_format, ragged_plan, full_plan):
+    announce(f"B{batch} H{heads} S{seq} D{dim} {kv_format}: {ragged_plan} and {full_plan}")
+    g = torch.Generator(device=DEV).manual_seed(7)
+    q = torch.randn((batch, heads, dim), generator=g, device=DEV, dtype=torch.float16)
+    k, v = (torch.randn((batch, heads, seq, dim), generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    lengths = torch.randint(1, seq + 1, (batch,), generator=torch.Generator().manual_seed(batch))
+    lengths[:3] = torch.tensor([seq, 0, 17])
+    cache = fa.PagedKVCache.from_dense(k, v, 16, lengths=lengths, block_table_pattern="interleaved", kv_format=kv_format)
+    kd, vd = cache.to_dense()
+    want = torch.zeros((batch, heads, dim), dtype=torch.float64, device=DEV)
+    for b, n in enumerate(lengths.tolist()):
+        if n:
+            scores = (kd[b, :, :n].double() * q[b, :, None].double()).sum(-1) / math.sqrt(dim)
+            want[b] = (vd[b, :, :n].double() * torch.softmax(scores, -1)[..., None]).sum(1)
+    cus = triton_utils.device_cu_count(DEV)
+    for full, plan in ((False, ragged_plan), (True, full_plan)):
+        got, st = fa.paged_quant_attention_triton(q, dataclasses.replace(cache, full_rows=full), return_stats=True)
+        if cus == 256:
+            assert (st["num_splits"], st["num_warps"]) == plan
+        assert torch.count_nonzero(got[1]).item() == 0  # the empty row
+        keep = [b for b in range(batch) if b != 1]
+        assert_attention_close(got[keep], want[keep].cpu().numpy(), torch.float16, f"{kv_format} full_rows={full}")

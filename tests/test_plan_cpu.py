@@ -16,10 +16,10 @@ from flashspec_amd.triton_utils import plan_rows
     (128, 8, True, 2), (64, 8, True, 4), (128, 8, True, 8), (128, 8, True, 64)])
 def test_plans_cover_the_row_within_the_limits(head_dim, max_waves, per_channel, group):
     for seq_len in (1, 16, 17, 300, 1024, 4095, 4096, 9000, 65536, 200000):
-        for rows in (1, 7, 24, 96, 128, 129, 160, 192, 255, 256, 257, 511, 512, 5000):
-            for light in (False, True):
+        for rows in (1, 7, 24, 72, 88, 96, 113, 114, 128, 129, 160, 192, 255, 256, 257, 511, 512, 5000):
+            for light, full_rows in ((False, False), (True, False), (False, True), (True, True)):
                 split, n, waves = plan_rows(seq_len, rows, head_dim, 256, max_waves=max_waves, tile_group=group,
-                                            light=light, per_channel=per_channel)
+                                            light=light, per_channel=per_channel, full_rows=full_rows)
                 tiles = -(-seq_len // 16)
                 assert split >= 1 and n >= 1 and waves in (1, 2, 4, 8, 16) and waves <= max_waves
                 assert split * n >= tiles > split * (n - 1)  # whole row, no empty split
@@ -39,6 +39,34 @@ def test_plans_at_the_lines_of_the_rule():
     assert plan(512, 64, 256, max_waves=8) == (16, 2, 4) and plan(512, 64) == (32, 1, 8)
 
 
+def test_plans_of_rows_that_leave_cus_idle():
+    def plan(tiles, rows, d=128, **kw):
+        return plan_rows(16 * tiles, rows, d, 256, max_waves=8 if d > 128 or kw.get("per_channel") else 16, **kw)
+
+    for full in (False, True):  # over half of the CUs: three splits, two of short rows, whole long and costly ones
+        assert plan(512, 170, full_rows=full) == (171, 3, 4) and plan(511, 171, full_rows=full) == (256, 2, 4)
+        assert plan(512, 171, full_rows=full) == (512, 1, 16) and plan(512, 255, full_rows=full) == (512, 1, 16)
+        assert plan(256, 192, 256, full_rows=full) == (256, 1, 8)
+        assert plan(256, 192, per_channel=True, full_rows=full) == (256, 1, 8)
+        assert plan(1024, 128, full_rows=full) == (512, 2, 16) and plan(1022, 128, full_rows=full) == (511, 2, 8)
+    # rows of unlike length take more workgroups than CUs where that was measured to gain
+    chan = {"per_channel": True}
+    assert plan(96, 96, **chan) == (32, 3, 8) and plan(96, 96, full_rows=True, **chan) == (48, 2, 8)
+    assert plan(95, 96, **chan) == (48, 2, 8) and plan(256, 80, **chan) == (86, 3, 8)
+    assert plan(256, 52, **chan) == (52, 5, 8) and plan(256, 60, **chan) == (64, 4, 8)
+    assert plan(256, 48, **chan) == (43, 6, 8) and plan(256, 48, full_rows=True, **chan) == (52, 5, 8)
+    assert plan(256, 144, **chan) == (128, 2, 8) and plan(256, 144, full_rows=True, **chan) == (86, 3, 4)
+    assert plan(256, 88, 256) == (86, 3, 8) and plan(256, 96, 256) == (128, 2, 8)
+    assert plan(256, 88, 256, full_rows=True) == (128, 2, 8)
+    assert plan(511, 102) == (256, 2, 8) and plan(512, 102) == (103, 5, 4) and plan(512, 103) == (256, 2, 8)
+    assert plan(512, 102, full_rows=True) == (256, 2, 8)
+    assert plan(768, 113) == (256, 3, 16) and plan(768, 114) == (384, 2, 8) and plan(768, 96, 64) == (154, 5, 8)
+    # light tiles on 4 waves: every CU, or nearly every one with full rows
+    assert plan(512, 120, light=True) == (256, 2, 8) and plan(510, 120, light=True, full_rows=True) == (255, 2, 4)
+    assert plan(512, 120, light=True, full_rows=True) == (256, 2, 8)
+    assert plan(16, 256, light=True) == (16, 1, 4) and plan(16, 256) == (16, 1, 8)
+
+
 @pytest.fixture()
 def launch_plan(monkeypatch):
     """triton_utils.launch_plan for a GPU of 256 CUs with no knob set, and a setter of knobs."""
@@ -50,8 +78,8 @@ def launch_plan(monkeypatch):
         monkeypatch.delenv(key, raising=False)
     monkeypatch.setitem(triton_utils._CU_CACHE, 0, 256)
     triton_utils._launch_plan_cached.cache_clear()
-    yield (lambda seq, rows, dim=128, **kw: triton_utils.launch_plan(seq, rows, dim, 16, 16, torch.device("cuda", 0), **kw),
-           monkeypatch.setenv)
+    dev = torch.device("cuda", 0)
+    yield lambda seq, rows, dim=128, **kw: triton_utils.launch_plan(seq, rows, dim, 16, 16, dev, **kw), monkeypatch.setenv
     triton_utils._launch_plan_cached.cache_clear()
 
 
@@ -75,3 +103,16 @@ def test_knobs_that_force_a_plan_still_do(launch_plan):
     assert plan(4096, 96)[1] == 4
     setenv("FLASHSPEC_NUM_SPLITS", "4")
     assert plan(4096, 96)[1:4] == (4, 64, 4)
+
+
+def test_caches_built_on_the_host_know_whether_their_rows_are_full():
+    from flashspec_amd import PagedKVCache
+
+    k = torch.zeros((4, 2, 32, 16))
+    full = lambda lengths: PagedKVCache.from_dense(k, k, 16, lengths=lengths).full_rows  # noqa: E731
+    assert full(None) and full(torch.tensor([32, 32, 32, 0])) and not full(torch.tensor([32, 32, 31, 0]))
+    cache = PagedKVCache.from_dense(k, k, 16)
+    assert not PagedKVCache(cache.k_quant, cache.v_quant, cache.block_table, cache.lengths, 16, 32).full_rows
+    for bad in ([33, 1, 1, 1], [1, -1, 1, 1], [1, 1, 1]):
+        with pytest.raises(ValueError):
+            full(torch.tensor(bad))
