@@ -480,14 +480,21 @@ _PLAN_KNOBS = ("FLASHSPEC_NUM_WARPS", "FLASHSPEC_BLOCK_N", "FLASHSPEC_NUM_SPLITS
 
 def _knob_reader():
     """A function that returns the knobs' values as they are now: os.environ's own mapping, read without
-    its per-lookup encoding where this Python has it (3 lookups: 1.2 us through os.environ.get, 0.15 us so)."""
+    its per-lookup encoding where this Python has it (3 lookups: 1.2 us through os.environ.get, 0.15 us so),
+    as long as os.environ is still that object."""
 
     env = os.environ
     data, encode = getattr(env, "_data", None), getattr(env, "encodekey", None)
     if not isinstance(data, dict) or encode is None:
-        return lambda: tuple([env.get(k) for k in _PLAN_KNOBS])
+        return lambda: tuple([os.environ.get(k) for k in _PLAN_KNOBS])
     a, b, c = (encode(k) for k in _PLAN_KNOBS)
-    return lambda: (data.get(a), data.get(b), data.get(c))
+
+    def read():
+        if os.environ is not env or env._data is not data:
+            return tuple([os.environ.get(k) for k in _PLAN_KNOBS])
+        return data.get(a), data.get(b), data.get(c)
+
+    return read
 
 
 _knobs = _knob_reader()

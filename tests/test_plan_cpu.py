@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import math
+import os
 
 import pytest
 import torch
@@ -103,6 +104,15 @@ def test_knobs_that_force_a_plan_still_do(launch_plan):
     assert plan(4096, 96)[1] == 4
     setenv("FLASHSPEC_NUM_SPLITS", "4")
     assert plan(4096, 96)[1:4] == (4, 64, 4)
+
+
+def test_knobs_are_read_from_the_environ_in_place(launch_plan, monkeypatch):
+    plan, _ = launch_plan
+    assert plan(4096, 96)[3] == 2
+    monkeypatch.setattr(os, "environ", {**os.environ, "FLASHSPEC_NUM_SPLITS": "4"})
+    assert plan(4096, 96)[3] == 4
+    os.environ["FLASHSPEC_NUM_SPLITS"] = "3"
+    assert plan(4096, 96)[3] == 3
 
 
 def test_caches_built_on_the_host_know_whether_their_rows_are_full():
