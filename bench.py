@@ -372,34 +372,37 @@ def quantize_bench(torch, fa, dev, calls: int = 30) -> dict:
 
 
 def page_quantize_bench(torch, fa, dev, calls: int = 30) -> dict:
-    """``PagedKVCache.from_dense``'s page quantizer (``fs_quantize_pages_i8``, one launch per tensor)
-    on one fp16 K tensor of the metric workload ([8, 32, 4096, 128] into 2048 16-token pages), in the
-    contiguous and the shuffled page order, input resident in HBM and rotated over two tensors;
+    """``PagedKVCache.from_dense``'s quantizer (``fs_build_cache``: K, V, block table and lengths in one
+    launch) on fp16 K and V of the metric workload ([8, 32, 4096, 128] into 2048 16-token pages), in
+    the contiguous and the shuffled page order, inputs resident in HBM and rotated over two pairs;
     bytes = fp16 read + int8 write + scale/zero write.  Beside it the same 2:1 copy ceiling as the
-    blocks quantizer's (`fs_stream_copy_half` over the same tensor, best grid)."""
+    blocks quantizer's (`fs_stream_copy_half` over one of the tensors, best grid)."""
 
     from flashspec_amd import _lib
 
     lib = _lib.require()
     g = torch.Generator(device=dev)
     g.manual_seed(6)
-    xs = [torch.randn((B, H, S, D), generator=g, device=dev, dtype=torch.float16) for _ in range(2)]
+    xs = [torch.randn((B, H, S, D), generator=g, device=dev, dtype=torch.float16) for _ in range(4)]
     pages = B * (S // PAGE)
-    values = torch.empty((pages, H, 1, PAGE, D), dtype=torch.int8, device=dev)
-    scale = torch.empty((pages, H, 1, 1, 1), dtype=torch.float32, device=dev)
-    zero = torch.empty((pages, H, 1, 1, 1), dtype=torch.int16, device=dev)
+    stores = [t for _ in range(2) for t in (torch.empty((pages, H, 1, PAGE, D), dtype=torch.int8, device=dev),
+                                            torch.empty((pages, H, 1, 1, 1), dtype=torch.float32, device=dev),
+                                            torch.empty((pages, H, 1, 1, 1), dtype=torch.int16, device=dev))]
+    table = torch.empty((B, S // PAGE), dtype=torch.int64, device=dev)
+    lengths = torch.empty((B,), dtype=torch.int64, device=dev)
     stream = _lib.stream_ptr(dev)
     gp = torch.Generator(device=dev)
     gp.manual_seed(0)
     perm = torch.randperm(pages, generator=gp, device=dev)
-    nbytes = B * H * S * D * (2 + 1) + pages * H * 6
-    out = {"workload": f"fs_quantize_pages_i8 fp16 [{B}, {H}, {S}, {D}] -> {pages} pages of {PAGE} tokens",
+    nbytes = 2 * (B * H * S * D * (2 + 1) + pages * H * 6) + 8 * (pages + B)
+    out = {"workload": f"fs_build_cache fp16 K and V [{B}, {H}, {S}, {D}] -> {pages} pages of {PAGE} tokens",
            "algorithmic_bytes": nbytes}
     for name, src in (("contiguous", None), ("shuffled", perm)):
         def call(i, src=src):
-            _lib.check(lib.fs_quantize_pages_i8(
-                xs[i % 2].data_ptr(), 1, B, H, S, D, PAGE, _lib.ptr(src), pages, values.data_ptr(),
-                scale.data_ptr(), zero.data_ptr(), stream))
+            k, v = xs[2 * (i % 2)], xs[2 * (i % 2) + 1]
+            _lib.check(lib.fs_build_cache(
+                k.data_ptr(), v.data_ptr(), 1, 0, B, H, S, D, PAGE, _lib.ptr(src), 0, pages,
+                *(t.data_ptr() for t in stores), table.data_ptr(), lengths.data_ptr(), stream))
         ms = time_loop(torch, call, calls, 3)
         gbps = nbytes / (ms * 1e-3) / 1e9
         out[name] = {"us_per_call": round(ms * 1e3, 2), "gbps": round(gbps, 1),
@@ -417,7 +420,7 @@ def page_quantize_bench(torch, fa, dev, calls: int = 30) -> dict:
                            "gbps": round(copy_gbps, 1), "workgroups": best[1]}
     for name in ("contiguous", "shuffled"):
         out[name]["frac_of_copy_ceiling"] = round(out[name]["gbps"] / copy_gbps, 4)
-    del xs, dst, values, scale, zero
+    del xs, dst, stores
     return out
 
 

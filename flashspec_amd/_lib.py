@@ -90,11 +90,6 @@ _SIGNATURES = {
         [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
          c_void_p],
     ),
-    "fs_quantize_pages_sym_i8": (
-        c_int,
-        [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
-         c_void_p],
-    ),
     "fs_build_cache": (
         c_int,
         [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int64, c_void_p,

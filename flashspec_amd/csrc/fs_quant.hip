@@ -1488,14 +1488,6 @@ extern "C" int fs_quantize_pages_i8_channel(const void* x, int x_dtype, int batc
                       PageStore{}, (hipStream_t)stream);
 }
 
-extern "C" int fs_quantize_pages_sym_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
-                                        int page_size, const int64_t* page_src, int64_t num_pages, int8_t* values,
-                                        float* scale, int16_t* zero, void* stream) {
-  return launch_pages<kGfToken>("quantize_pages_symmetric", x, nullptr, x_dtype, batch, heads, seq_len, head_dim, page_size,
-                      PagePlan{page_src, 0, num_pages, nullptr, nullptr}, PageStore{values, scale, zero},
-                      PageStore{}, (hipStream_t)stream);
-}
-
 extern "C" int fs_build_cache(const void* k, const void* v, int src_dtype, int kv_format, int batch, int heads,
                               int seq_len, int head_dim, int page_size, const int64_t* page_src, int interleaved,
                               int64_t num_pages, void* k_values, float* k_scale, int16_t* k_zero, void* v_values,

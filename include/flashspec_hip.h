@@ -329,16 +329,10 @@ int fs_quantize_i8(const void* x, int x_dtype, int64_t outer, int seq_len, int h
  */
 int fs_quantize_sym_i8(const void* x, int x_dtype, int64_t rows, int head_dim,
                        int8_t* values, float* scale, int16_t* zero, void* stream);
-/* The same quantizer over the pages of dense [batch, heads, seq_len, head_dim] values, placed as
- * fs_quantize_pages_i8 places them: values [num_pages, heads, page_size, head_dim], scale / zero
- * [num_pages, heads, page_size]; rows past seq_len are zero. */
-int fs_quantize_pages_sym_i8(const void* x, int x_dtype, int batch, int heads, int seq_len, int head_dim,
-                             int page_size, const int64_t* page_src, int64_t num_pages,
-                             int8_t* values, float* scale, int16_t* zero, void* stream);
-
 /* A whole paged cache from dense k and v [batch, heads, seq_len, head_dim] in one launch (replaces
  * reference paged.py:302-419): both stores as the fs_quantize_pages_* entry of kv_format (0 affine
- * INT8, 1 FP8 E4M3, 2 per-channel INT8, 3 symmetric per-token INT8) writes them, and, where not
+ * INT8, 1 FP8 E4M3, 2 per-channel INT8) writes them, or with 3 as fs_quantize_sym_i8 quantizes rows
+ * (scale / zero [num_pages, heads, page_size]; rows past seq_len are zero), and, where not
  * NULL, block_table [batch, ceil(seq_len / page_size)] and lengths [batch] (all seq_len).  Pages are
  * placed by page_src (physical page j holds batch-major logical page page_src[j], a permutation), or
  * without it in batch-major order, or with `interleaved` in logical-page-major order. */

@@ -301,6 +301,48 @@ def test_dequantize_matches_the_portable_path(dtype, dim, block, seq):
         assert torch.equal(got.cpu(), want)
 
 
+# the C entries that quantize one tensor, which the package itself reaches through fs_build_cache only
+@pytest.mark.parametrize("entry,kv_format", [("fs_quantize_pages_i8", "affine_block"),
+                                             ("fs_quantize_pages_fp8", "fp8_block"),
+                                             ("fs_quantize_pages_i8_channel", "affine_channel")])
+@pytest.mark.parametrize("dim", [128, 36])
+def test_page_quantizers_of_the_c_interface_match_a_built_cache(entry, kv_format, dim):
+    announce(f"{entry} D{dim}")
+    x = randn((3, 2, 50, dim), 6, torch.float16).to(DEV)
+    cache = fa.PagedKVCache.from_dense(x, x, 16, block_table_pattern="shuffled", layout_seed=5, kv_format=kv_format)
+    want = cache.k_quant
+    out = [torch.empty_like(t) for t in (want.values, want.scale, want.zero_point)]
+    src = torch.empty(12, dtype=torch.int64, device=DEV)
+    src[cache.block_table.reshape(-1)] = torch.arange(12, device=DEV)
+    _lib.check(getattr(_lib.require(), entry)(x.data_ptr(), _lib.dtype_code(x.dtype), 3, 2, 50, dim, 16, src.data_ptr(), 12,
+                                              *(t.data_ptr() for t in out), _lib.stream_ptr(DEV)))
+    assert_same_store(fa.QuantizedTensor(*out, want.block_size, want.original_shape), want, entry)
+
+
+def test_page_update_of_fresh_pages_ignores_what_they_held():
+    announce("fs_update_pages_i8 with fresh pages")
+    heads, page, dim = 2, 16, 32
+    old = fa.quantize_int8_per_block(randn((4, heads, page, dim), 7).to(DEV), page)
+    new = randn((1, heads, 3, dim), 8, torch.float16).to(DEV)
+    out = [t.clone() for t in (old.values, old.scale, old.zero_point)]
+    pages = torch.tensor([3, 1], device=DEV)
+    fresh = torch.tensor([1, 0], dtype=torch.uint8, device=DEV)
+    rows = torch.full((2, page), -1, dtype=torch.int32)
+    rows[0, :2], rows[1, 5] = torch.tensor([0, 1]), 2
+    held = fa.dequantize_int8_per_block(old).cpu().reshape(4, heads, page, dim)
+    held[3] = 0
+    held[3, :, :2], held[1, :, 5] = new[0, :, :2].float().cpu(), new[0, :, 2].float().cpu()
+    rows = rows.to(DEV)
+    _lib.check(_lib.require().fs_update_pages_i8(
+        *(t.data_ptr() for t in out), 4, page, *(t.data_ptr() for t in out), pages.data_ptr(), fresh.data_ptr(), 2,
+        rows.data_ptr(), new.data_ptr(), _lib.dtype_code(new.dtype), 3, heads, page, dim, _lib.stream_ptr(DEV)))
+    want = fa.quantize_int8_per_block(held, page)
+    for name, got, had, w in zip(("values", "scale", "zero"), out, (old.values, old.scale, old.zero_point),
+                                 (want.values, want.scale, want.zero_point)):
+        assert torch.equal(got[[0, 2]], had[[0, 2]]), name
+        assert torch.equal(got[[1, 3]].cpu(), w[[1, 3]]), name
+
+
 # a launch holds 2^26 - 4 groups of one wave: K's 40 million end inside the first, V's pass into a second
 LAUNCH_GROUPS = 4 * (2 ** 24 - 1)
 
