@@ -321,33 +321,34 @@ def plan_splits(seq_len: int, rows: int, block_n: int, cu_count: int, *, tiled: 
     return split_tiles, math.ceil(tiles / split_tiles), waves
 
 
-# The default plan of the tiled path (plan_splits serves forced counts).  Measured on MI355X, kernel time of
-# paged launches in us, 7 formats (INT8 with fp16 or fp32 queries, FP8, per-token, per-channel, head_dim 64
-# and 256), 1 to 640 rows of 8 to 1024 tiles, every row full or rows of unlike length ("ragged"; the figures
-# are the mean of 4 draws), splits x waves.  Figures are INT8, fp16 queries, 128 dims where no format is
-# named.
-# * A row takes at most sqrt(tiles) / 2 splits: the last split's merge grows with their number.  4 rows of
+# The default plan of the tiled path (plan_splits serves forced counts). Measured on MI355X, kernel time in
+# us, 7 formats (INT8 with fp16 or fp32 queries, FP8, per-token, per-channel, head_dim 64 and 256), 1 to 640
+# rows of 8 to 1024 tiles, paged (contiguous and shuffled pages) and contiguous, every row full or rows of
+# unlike length ("ragged"; the figures are the mean of 3 or 4 draws), splits x waves. Figures are INT8, fp16
+# queries, 128 dims, contiguous pages where nothing else is named.
+# * A row takes at most sqrt(tiles) / 2 splits: the last split's merge grows with their number. 4 rows of
 #   1024 tiles: 64 splits 29.0, 16 splits 16.0; 8 rows of 128 tiles: 16 splits 12.1, 5 splits 9.3.
 # * Rows under PLAN_MIN_TILES stay whole (64 rows of 32 tiles: 4 splits 7.8, unsplit 6.6); 256-dim and
 #   per-channel tiles, whose tiles cost about twice as much, from half of that.
 # * One round: splits that leave no workgroup for a second round, which costs a whole split (96 full rows of
-#   256 tiles: 3 x 16 32.1, 2 x 8 20.7).  8 waves per workgroup, two tiles a wave at least (four at 256 dims
-#   or with more rows than CUs), merged in the launch; 16 waves and a merge launch only where a wave of 8
-#   would hold 64 tiles (128 rows of 1024 tiles: 2 x 8 99.8, 2 x 16 89.5).
-# * That leaves CUs idle where rows do not divide them.  Whole rows on over half of the CUs take two
+#   256 tiles: 3 x 16 32.1, 2 x 8 20.7). 8 waves per workgroup, two tiles a wave at least (four at 256 dims
+#   or with more rows than CUs), merged in the launch: splits on 16 waves pay a workspace and a merge
+#   launch.
+# * That leaves CUs idle where rows do not divide them. Whole rows on over half of the CUs take two
 #   workgroups a CU from PLAN_SLOT_TILES on: three 4-wave splits (144 rows of 256 tiles: 1 x 16 30.3, 3 x 4
 #   30.5, ragged 27.9 and 23.6), or two below PLAN_WHOLE_TILES (224 rows of 256: 1 x 8 41.4, 2 x 4 42.4; 240
-#   ragged: 34.8 and 31.9).  From there on two 4-wave splits lose to the whole row on 16 waves (240 rows of
-#   512 tiles: 106.1 and 79.6), and costly tiles gain nothing from them at all (256 dims, 192 rows of 256: 2
-#   x 4 78.7, 1 x 8 63.8).
+#   ragged: 34.8 and 31.9). From there on two 4-wave splits lose to the whole row (208 rows of 512 tiles:
+#   contiguous pages 89.8 and 74.6, shuffled 73.9 and 70.2, contiguous store 70.8 and 66.9), but for ragged
+#   64-dim rows, on 8 waves (192 of 512: 1 x 8 35.8, 2 x 8 30.8); costly tiles gain nothing from them at all
+#   (256 dims, 192 rows of 256: 2 x 4 78.7, 1 x 8 63.8).
 # * Ragged rows leave some of their splits empty, so that a few workgroups too many cost them nothing
-#   (full_rows: the host knows that every row holds seq_len tokens).  One split more: per-channel tiles, 96
-#   rows of 512 (full 2 x 8 59.7, 3 x 8 79.5; ragged 56.3 and 46.1) and 52 rows (ragged 4 x 8 32.4, 5 x 8
-#   28.5), 256 dims where it is 4% over the CUs (88 rows of 256 tiles, ragged: 27.7 and 23.0).  Four splits
-#   in place of three gain nothing (80 rows, per-channel, 256 tiles, ragged: 3 x 8 24.8, 4 x 8 29.1).  Other
-#   tiles, two splits too few: two workgroups a CU from PLAN_WHOLE_TILES on (96 ragged rows of 512: 2 x 8
-#   30.5, 5 x 4 27.8), three splits of 16 waves from PLAN_DEEP_TILES (96 ragged rows of 1024: 2 x 8 53.0, 3
-#   x 16 44.9; not the 64-dim layout).
+#   (full_rows: the host knows that the rows are full). A third split within 4% of the CUs (88 ragged rows
+#   of 256 tiles: 2 x 8 17.5, 3 x 8 15.3) and a split more of per-channel tiles (96 rows of 512: full 2 x 8
+#   59.7, 3 x 8 79.5, ragged 56.3 and 46.1; 52 ragged rows of 512: 4 x 8 32.4, 5 x 8 28.5), but not four in
+#   place of three (80 ragged rows of 256: 24.8 and 29.1). Other rows with two splits too few: two
+#   workgroups a CU from PLAN_WHOLE_TILES on (96 ragged rows of 512: 2 x 8 30.5, 5 x 4 27.8), three splits
+#   of 16 waves from PLAN_DEEP_TILES (96 ragged rows of 1024: 2 x 8 53.0, 3 x 16 44.9; not the 64-dim
+#   layout).
 # * Light tiles (LIGHT_WAVES) take 4 waves where a workgroup lands on every CU and a wave keeps 16 to 64
 #   tiles (256 rows of 256 tiles: 42.1, on 8 waves 44.2), and with full rows on nearly every CU (48 rows of
 #   768: 5 x 4 29.4, 5 x 8 32.1; 120 ragged rows of 512 instead: 2 x 4 40.1, 2 x 8 31.6).
@@ -367,9 +368,9 @@ PLAN_LIGHT_FULL_ROWS_FILL = 0.9
 
 def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_waves: int = MAX_TILED_WAVES,
               tile_group: int = 1, light: bool = False, per_channel: bool = False,
-              full_rows: bool = False) -> tuple[int, int, int]:
+              full_rows: bool = True) -> tuple[int, int, int]:
     """``(split_tiles, max_splits, waves_per_block)`` of a tiled decode launch (rule above); arguments as
-    for ``plan_splits``.  ``full_rows``: as far as the host knows, every row holds ``seq_len`` tokens."""
+    for ``plan_splits``.  ``full_rows``: as far as the host knows, the rows hold (nearly) ``seq_len`` tokens each."""
 
     tiles = max(1, math.ceil(seq_len / TILE_TOKENS))
     grp = max(1, tile_group)
@@ -382,10 +383,11 @@ def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_wave
     side_by_side = deep = False  # two smaller workgroups a CU; splits of 16 waves with a merge launch
     if n == one_round and n * rows < cu_count:
         pairs = 2 * cu_count // rows
-        if costly and not full_rows and _ragged_costly_split(n, tiles, (n + 1) * rows / cu_count, per_channel):
+        if not full_rows and _one_more_split(n, tiles, (n + 1) * rows / cu_count, per_channel):
             n += 1
         elif n == 1 and tiles >= PLAN_SLOT_TILES:
-            side_by_side = pairs == 3 or (not costly and tiles < PLAN_WHOLE_TILES)
+            side_by_side = pairs == 3 or (not costly and (tiles < PLAN_WHOLE_TILES or
+                                                          (head_dim <= 64 and not full_rows)))
         elif n == 2 and not costly and not full_rows:
             deep = tiles >= PLAN_DEEP_TILES and head_dim > 64 and 9 * rows <= 4 * cu_count
             side_by_side = not deep and tiles >= PLAN_WHOLE_TILES and pairs > 4
@@ -406,7 +408,7 @@ def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_wave
     elif split >= LIGHT_MIN_SPLIT_TILES and (every_cu and split <= LIGHT_WAVES * MAX_TILES_PER_WAVE or
                                              nearly_every_cu and split < LIGHT_WAVES * MAX_TILES_PER_WAVE):
         waves = min(waves, LIGHT_WAVES)
-    elif deep or split >= PLAN_WHOLE_TILES or (rows >= cu_count and split >= PLAN_LONG_TILES):
+    elif deep or (rows >= cu_count and split >= PLAN_LONG_TILES):
         waves = max_waves
     while waves < max_waves and split_groups > MAX_TILES_PER_WAVE // grp * waves:
         waves *= 2
@@ -416,13 +418,15 @@ def plan_rows(seq_len: int, rows: int, head_dim: int, cu_count: int, *, max_wave
     return split_groups * grp, math.ceil(tiles / (split_groups * grp)), waves
 
 
-def _ragged_costly_split(n: int, tiles: int, over: float, per_channel: bool) -> bool:
-    """Whether ragged rows of costly tiles take a split more than the ``n`` of one round, which asks for
-    ``over`` times the CUs (rule above)."""
+def _one_more_split(n: int, tiles: int, over: float, per_channel: bool) -> bool:
+    """Whether rows of unlike length take a split more than the ``n`` of one round, which asks for ``over``
+    times the CUs (rule above)."""
 
-    if not per_channel:
-        return n == 2 and tiles >= PLAN_RAGGED_TILES and over <= 1.04
-    return (n == 2 and tiles >= PLAN_RAGGED_TILES) or (n != 3 and tiles >= 2 * PLAN_RAGGED_TILES and over <= 1.13)
+    if n == 2:
+        return tiles >= PLAN_RAGGED_TILES and (over <= 1.04 or per_channel)
+    # (whole rows on up to 2/3 of the CUs have three smaller splits to take instead)
+    return per_channel and n != 3 and tiles >= 2 * PLAN_RAGGED_TILES and \
+        (over <= 1.13 or (n == 1 and 4 / 3 < over <= 1.5))
 
 
 # One 8-wave workgroup of the multi-query kernel holds a CU (its ~140 registers per lane leave
@@ -480,7 +484,7 @@ _PLAN_KNOBS = ("FLASHSPEC_NUM_WARPS", "FLASHSPEC_BLOCK_N", "FLASHSPEC_NUM_SPLITS
 
 def _knob_reader():
     """A function that returns the knobs' values as they are now: os.environ's own mapping, read without
-    its per-lookup encoding where this Python has it (3 lookups: 1.2 us through os.environ.get, 0.15 us so),
+    its per-lookup encoding where this Python has it (3 lookups: 1.2 us through os.environ.get, a tenth of that so),
     as long as os.environ is still that object."""
 
     env = os.environ
@@ -501,7 +505,7 @@ _knobs = _knob_reader()
 
 
 def launch_plan(seq_len: int, rows: int, head_dim: int, page_size: int, quant_block: int, device,
-                per_channel: bool = False, light: bool = False, contiguous: bool = False, full_rows: bool = False):
+                per_channel: bool = False, light: bool = False, contiguous: bool = False, full_rows: bool = True):
     """(tiled, waves_per_block, split_tiles, max_splits, block_n) for one decode launch.
 
     ``light``: fp16 or bf16 query over INT8 or FP8 values (the caller's part of the LIGHT_WAVES condition;

@@ -240,14 +240,14 @@ def test_stale_merge_words_from_earlier_launches_are_not_taken(monkeypatch):
 # one call on each side of the default plan's lines for rows that leave CUs idle: a split more than one
 # round holds, two workgroups a CU, 16-wave splits (merge launch), whole rows
 @pytest.mark.parametrize("batch,heads,seq,dim,kv_format,ragged_plan,full_plan", [
-    (11, 8, 12288, 128, "affine_block", (3, 16), (2, 8)),
+    (12, 8, 12288, 128, "affine_block", (3, 16), (2, 8)),
     (12, 8, 8192, 128, "fp8_block", (5, 4), (2, 8)),
     (12, 8, 8192, 64, "affine_block", (5, 8), (2, 8)),
     (12, 8, 1536, 128, "affine_channel", (3, 8), (2, 8)),
     (11, 8, 1536, 256, "affine_block", (3, 8), (2, 8)),
     (6, 8, 4090, 128, "affine_channel", (6, 8), (5, 8)),
     (18, 8, 4096, 64, "symmetric_token", (3, 8), (3, 4)),
-    (24, 8, 8192, 128, "affine_block", (1, 16), (1, 16)),
+    (24, 8, 8192, 64, "affine_block", (2, 8), (1, 8)),
 ])
 def test_default_plans_of_rows_that_leave_cus_idle(batch, heads, seq, dim, kv_format, ragged_plan, full_plan):
     announce(f"B{batch} H{heads} S{seq} D{dim} {kv_format}: {ragged_plan} and {full_plan}")

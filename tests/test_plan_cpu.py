@@ -41,15 +41,17 @@ def test_plans_at_the_lines_of_the_rule():
 
 
 def test_plans_of_rows_that_leave_cus_idle():
-    def plan(tiles, rows, d=128, **kw):
-        return plan_rows(16 * tiles, rows, d, 256, max_waves=8 if d > 128 or kw.get("per_channel") else 16, **kw)
+    def plan(tiles, rows, d=128, full_rows=False, **kw):
+        return plan_rows(16 * tiles, rows, d, 256, max_waves=8 if d > 128 or kw.get("per_channel") else 16,
+                         full_rows=full_rows, **kw)
 
     for full in (False, True):  # over half of the CUs: three splits, two of short rows, whole long and costly ones
         assert plan(512, 170, full_rows=full) == (171, 3, 4) and plan(511, 171, full_rows=full) == (256, 2, 4)
-        assert plan(512, 171, full_rows=full) == (512, 1, 16) and plan(512, 255, full_rows=full) == (512, 1, 16)
+        assert plan(512, 171, full_rows=full) == (512, 1, 8) and plan(513, 255, full_rows=full) == (513, 1, 16)
         assert plan(256, 192, 256, full_rows=full) == (256, 1, 8)
-        assert plan(256, 192, per_channel=True, full_rows=full) == (256, 1, 8)
-        assert plan(1024, 128, full_rows=full) == (512, 2, 16) and plan(1022, 128, full_rows=full) == (511, 2, 8)
+        assert plan(256, 193, per_channel=True, full_rows=full) == (256, 1, 8)
+        assert plan(1024, 128, full_rows=full) == (512, 2, 8)
+    assert plan(512, 192, 64) == (256, 2, 8) and plan(512, 192, 64, full_rows=True) == (512, 1, 8)
     # rows of unlike length take more workgroups than CUs where that was measured to gain
     chan = {"per_channel": True}
     assert plan(96, 96, **chan) == (32, 3, 8) and plan(96, 96, full_rows=True, **chan) == (48, 2, 8)
@@ -57,8 +59,10 @@ def test_plans_of_rows_that_leave_cus_idle():
     assert plan(256, 52, **chan) == (52, 5, 8) and plan(256, 60, **chan) == (64, 4, 8)
     assert plan(256, 48, **chan) == (43, 6, 8) and plan(256, 48, full_rows=True, **chan) == (52, 5, 8)
     assert plan(256, 144, **chan) == (128, 2, 8) and plan(256, 144, full_rows=True, **chan) == (86, 3, 4)
-    assert plan(256, 88, 256) == (86, 3, 8) and plan(256, 96, 256) == (128, 2, 8)
-    assert plan(256, 88, 256, full_rows=True) == (128, 2, 8)
+    assert plan(256, 192, **chan) == (128, 2, 8) and plan(256, 192, full_rows=True, **chan) == (256, 1, 8)
+    for dim in (64, 128, 256):
+        assert plan(96, 88, dim) == (32, 3, 8) and plan(96, 88, dim, full_rows=True) == (48, 2, 8)
+        assert plan(256, 96, dim) == (128, 2, 8)
     assert plan(511, 102) == (256, 2, 8) and plan(512, 102) == (103, 5, 4) and plan(512, 103) == (256, 2, 8)
     assert plan(512, 102, full_rows=True) == (256, 2, 8)
     assert plan(768, 113) == (256, 3, 16) and plan(768, 114) == (384, 2, 8) and plan(768, 96, 64) == (154, 5, 8)
@@ -80,7 +84,8 @@ def launch_plan(monkeypatch):
     monkeypatch.setitem(triton_utils._CU_CACHE, 0, 256)
     triton_utils._launch_plan_cached.cache_clear()
     dev = torch.device("cuda", 0)
-    yield lambda seq, rows, dim=128, **kw: triton_utils.launch_plan(seq, rows, dim, 16, 16, dev, **kw), monkeypatch.setenv
+    yield (lambda seq, rows, dim=128, **kw: triton_utils.launch_plan(seq, rows, dim, 16, 16, dev, **kw),
+           monkeypatch.setenv)
     triton_utils._launch_plan_cached.cache_clear()
 
 
