@@ -1034,8 +1034,10 @@ tree_prefix_mfma_kernel(const DecodeParams p) {
     // four dims a thread; rows that need nothing more (one split, draft tokens already in the states) go
     // out from here.  With one float a thread and the rows through s_fin the merge took twice as many
     // LDS instructions and a barrier more per node group, of a workgroup's ~12 us beside its tiles.
-    // Measured, H32 D128: B8 x 64 nodes fp16 over 1024 tokens 43.1 -> 40.1 us, bf16 over 4096 112.2 ->
-    // 110.4, B4 x 16 over 4096 34.0 -> 33.6; 256 dims, B4 x 16 over 2048, 44.7 -> 42.7.
+    // Measured, H32 D128, both builds in turn: B8 x 64 nodes over 1024 tokens fp16 45.7 -> 42.6 us, bf16
+    // (rows do not go out from here: drafts other than fp16 walk their paths after) 53.4 -> 51.1; 256 dims,
+    // B4 x 16 over 2048, 44.6 -> 42.9.  Over 4096 tokens B4 x 16 34.0 -> 33.7 (runs differ by 0.4), B8 x 64
+    // bf16 106 -> 104 to 106: within the spread.
     const bool direct = p.fuse_tail && !merge_here && draft_mfma;
     constexpr int QD = DP / 4;
     for (int e = threadIdx.x; e < nodes_here * QD; e += blockDim.x) {
