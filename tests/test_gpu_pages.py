@@ -401,6 +401,21 @@ def test_block_quantizer_of_more_groups_than_one_launch_holds():
         assert torch.equal(got, want)
 
 
+def test_to_dense_of_more_rows_than_32_bits_count():
+    n, pages = 2 ** 30 + 7, 1000  # K and V: 2^31 + 14 rows of one value, each its own wave
+    announce(f"to_dense of {n} one-token pages of one value")
+    g = torch.Generator(device=DEV).manual_seed(6)
+    k, v = (fa.quantize_int8_per_block(torch.randn((pages, 1, 1, 1), generator=g, device=DEV), 1) for _ in range(2))
+    table = torch.randint(0, pages, (1, n), generator=g, device=DEV, dtype=torch.int32)
+    lengths = torch.tensor([n], device=DEV)
+    dense = fa.PagedKVCache(k, v, table, lengths, 1, n).to_dense()
+    for q, d in zip((k, v), dense):
+        assert d.shape == (1, 1, n, 1)
+        page = fa.dequantize_int8_per_block(q).reshape(pages)
+        for at in range(0, n, 1 << 27):
+            assert torch.equal(d[0, 0, at:at + (1 << 27), 0], page[table[0, at:at + (1 << 27)].long()]), at
+
+
 def test_token_quantizer_of_more_rows_than_one_launch_holds():
     n, dim = LAUNCH_GROUPS + 5, 4  # a wave per row
     announce(f"quantize_int8_symmetric_per_token of {n} rows")
