@@ -322,6 +322,7 @@ class PagedKVAllocator:
             lengths=lengths.to(self.device),
             block_size=self.block_size,
             max_seq_len=int(lengths.max().item()),
+            full_rows=rows_mostly_full(lengths.tolist(), int(lengths.max().item())),
         )
 
     def stats(self) -> Dict[str, float]:
@@ -406,6 +407,12 @@ def _layout_permutation(pattern: str, batch: int, blocks_per_seq: int, layout_se
     return None
 
 
+def rows_mostly_full(lengths: Sequence[int], span: int) -> bool:
+    """Whether rows of these lengths fill at least 3/4 of their ``span`` on average (``full_rows``)."""
+
+    return 4 * sum(lengths) >= 3 * len(lengths) * span
+
+
 @dataclass(frozen=True)
 class PagedKVCache:
     """Paged INT8 KV cache (paged.py:258-300).
@@ -483,7 +490,7 @@ class PagedKVCache:
             held = effective_lengths.tolist()
             if any(not 0 <= n <= seq_len for n in held):
                 raise ValueError("lengths must lie in [0, seq_len]")
-            full_rows = 4 * sum(held) >= 3 * batch * seq_len
+            full_rows = rows_mostly_full(held, seq_len)
 
         if on_gpu:
             k_quant, v_quant, block_table, full_lengths = cls._build_hip(k, v, block_size, perm,
@@ -672,6 +679,7 @@ class PagedKVCache:
             k_quant=new_stores[0], v_quant=new_stores[1],
             block_table=torch.from_numpy(table).to(dev), lengths=torch.from_numpy(lengths).to(dev),
             block_size=bs, max_seq_len=int(lengths.max()),
+            full_rows=rows_mostly_full(lengths.tolist(), int(lengths.max())),
         )
 
     def _append_portable(self, k_new: torch.Tensor, v_new: torch.Tensor, tokens: int) -> "PagedKVCache":
@@ -702,6 +710,7 @@ class PagedKVCache:
             block_table=torch.from_numpy(table_np).to(device),
             lengths=torch.from_numpy(lengths_np).to(device),
             block_size=bs, max_seq_len=int(lengths_np.max()),
+            full_rows=rows_mostly_full(lengths_np.tolist(), int(lengths_np.max())),
         )
 
     def estimated_bytes(self) -> int:

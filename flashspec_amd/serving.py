@@ -34,7 +34,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .paged import PagedKVAllocator, PagedKVCache
+from .paged import PagedKVAllocator, PagedKVCache, rows_mostly_full
 from .quant import QuantizedTensor, dequantize_int8_per_block, quantize_int8_per_block
 from .runtime import device_name, resolve_device, resolve_dtype, synchronize
 from .triton_paged import _run_paged_quant_attention_triton, paged_quant_attention_triton
@@ -350,7 +350,7 @@ class DecodeBatch:
         if cached is None or cached[0] != key:
             cached = (key, PagedKVCache(k_quant=self.allocator.k_quant, v_quant=self.allocator.v_quant,
                                         block_table=self.block_table, lengths=self.lengths, block_size=self.page,
-                                        max_seq_len=cap))
+                                        max_seq_len=cap, full_rows=rows_mostly_full(self.host_lengths, cap)))
             self._caches[self._cur] = cached
         return cached[1]
 

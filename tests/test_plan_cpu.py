@@ -121,12 +121,22 @@ def test_knobs_are_read_from_the_environ_in_place(launch_plan, monkeypatch):
 
 
 def test_caches_built_on_the_host_know_whether_their_rows_are_full():
-    from flashspec_amd import PagedKVCache
+    from flashspec_amd import PagedKVAllocator, PagedKVCache
 
     k = torch.zeros((4, 2, 32, 16))
     full = lambda lengths: PagedKVCache.from_dense(k, k, 16, lengths=lengths).full_rows  # noqa: E731
     assert full(None) and full(torch.tensor([32, 32, 32, 0])) and not full(torch.tensor([32, 32, 31, 0]))
     cache = PagedKVCache.from_dense(k, k, 16)
+    step = torch.zeros((4, 2, 1, 16))
+    assert cache.append(step, step).full_rows
+    assert not PagedKVCache.from_dense(k, k, 16, lengths=torch.tensor([32, 1, 1, 1])).append(step, step).full_rows
+    pool = PagedKVAllocator(capacity_blocks=16, heads=2, head_dim=16)
+    for rid, n in enumerate((32, 30, 2)):
+        pool.add_request(rid, k[:1, :, :n], k[:1, :, :n])
+    assert pool.to_cache([0, 1]).full_rows and not pool.to_cache([0, 2]).full_rows
+    old = PagedKVCache.from_dense(k, k, 16)
+    del old.__dict__["full_rows"]  # as unpickled from before the field
+    assert not old.full_rows
     assert not PagedKVCache(cache.k_quant, cache.v_quant, cache.block_table, cache.lengths, 16, 32).full_rows
     for bad in ([33, 1, 1, 1], [1, -1, 1, 1], [1, 1, 1]):
         with pytest.raises(ValueError):
