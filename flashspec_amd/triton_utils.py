@@ -494,7 +494,7 @@ def _knob_reader():
     a, b, c = (encode(k) for k in _PLAN_KNOBS)
 
     def read():
-        if os.environ is not env or env._data is not data:
+        if os.environ is not env:
             return tuple([os.environ.get(k) for k in _PLAN_KNOBS])
         return data.get(a), data.get(b), data.get(c)
 
