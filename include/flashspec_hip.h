@@ -489,7 +489,7 @@ int fs_write_prompt_i8(const void* k, const void* v, int src_dtype, int src_toke
  * then dropped and nothing is written).  `dropped` (NULL, or one unsigned of device memory the
  * caller zeroes) counts the dropped tokens, one per request, with device atomics: the reference
  * allocator raises instead of dropping (paged.py:89-90, 222-224), so a caller that must not lose
- * tokens checks it.  lengths_in and lengths_out must differ; the caller
+ * tokens checks it.  batch * heads is at most 2^25 - 2.  lengths_in and lengths_out must differ; the caller
  * fills the table entry of a page before the step that first writes it.
  * Replaces PagedKVAllocator.append_batch for one token per request
  * (reference src/flashspec/paged.py:108-144, with page reads at :226-245 and writes at :247-255). */
